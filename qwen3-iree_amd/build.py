@@ -101,7 +101,7 @@ def build_shim() -> Path:
 OBJECT_SOURCES = {
     "q8gemv": ("q8gemv_kernels.hip", "q8_device.h"),
     "decode": ("decode_kernels.hip", "decode_device.h", "q8_device.h"),
-    "prefill": ("prefill_kernels.hip", "prefill_split.h", "decode_device.h", "q8_device.h"),
+    "prefill": ("prefill_kernels.hip", "prefill_rows.h", "prefill_split.h", "decode_device.h", "q8_device.h"),
 }
 
 

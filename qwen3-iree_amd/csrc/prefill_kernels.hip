@@ -17,8 +17,10 @@
 //   pf_gemm_q8       gate/up with SwiGLU in the epilogue
 //   pf_gemm_q8       ffn_down + residual
 // plus pf_embed (token rows) before the first layer.  The vocab GEMV + argmax
-// of the last token reuses the decode kernels.  Prompts below 1024 tokens run
-// attn_o and ffn_down with K split (pf_gemm_q8_part); their reduce
+// of the last token reuses the decode kernels.  Up to 128 tokens the products
+// and norms are five launches of prefill_rows.h (four from 65 tokens on, with
+// RoPE in the q/k/v one, which runs up to 256).  Prompts of 129 to 1023 tokens
+// run attn_o and ffn_down with K split (pf_gemm_q8_part); their reduce
 // (pf_res_reduce_norm) then also forms the rms_norm that follows (ffn_norm of
 // the row after attn_o, the next layer's attn_norm after ffn_down), so those
 // two pf_rmsnorm launches drop out.
@@ -30,8 +32,8 @@
 // converter makes from a Q8_0 file, f16(scale * q) with the product exact in
 // f32 and rounded once (tools/convert_gguf_to_irpa.py:28-44, 174-199); every
 // weight is formed that way in registers (one f16 multiply of the exact
-// integer q by the f16 scale) and the MFMA accumulates f16 x * f16 w in f32
-// over the whole K.
+// integer q by the f16 scale) and the MFMA accumulates f16 x * f16 w in f32,
+// over the whole K or over K ranges whose sums are added in order in f32.
 #include "decode_device.h"
 #include "prefill_split.h"
 
@@ -753,6 +755,8 @@ extern "C" __global__ __launch_bounds__(64) void pf_rope_table(int start, float*
   table[(size_t)i * 128 + lane] = c;
   table[(size_t)i * 128 + 64 + lane] = s;
 }
+
+#include "prefill_rows.h"
 
 // Token i = blockIdx.x (position start + i): per-head rms_norm with q_norm /
 // k_norm (qwen3_full.mlir:1812-1879) and RoPE (@position_components.rope,

@@ -129,6 +129,10 @@ struct State {
                 pf_f16_res_22 = nullptr, pf_f16_res_22k = nullptr, pf_f16_res_12k = nullptr,
                 pf_f16_part_22 = nullptr, pf_f16_part_22k = nullptr, pf_f16_part_12k = nullptr,
                 pf_f16_part_44 = nullptr, pf_f16_part_44k = nullptr, pf_expand = nullptr;
+  // the row products (prefill_rows.h): [instance, fewest tokens first][0: f16
+  // weights, 1: Q8_0]
+  hipFunction_t pf_rows_qkv_rope[2][2] = {}, pf_rows_qkv[2][2] = {}, pf_rows_gu[4][2] = {},
+                pf_rows_o[2][2] = {}, pf_rows_dn[2][2] = {};
   std::atomic<int> pf_tile_rows{0};   // prefill GEMM token tile: 0 = by shape, 32, 64 or 128
   std::atomic<int> pf_attn_split{0};  // prefill attention positions per split in blocks of 32
   std::atomic<int> step_single{-1};   // single-launch decode step: -1 unknown, 0 off, 1 on
@@ -387,6 +391,30 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_f16_part_12k, "pf_gemm_f16_part_12k"},
                      {&g.pf_f16_part_44, "pf_gemm_f16_part_44"},
                      {&g.pf_f16_part_44k, "pf_gemm_f16_part_44k"},
+                     {&g.pf_rows_qkv_rope[0][0], "pf_rows_qkv_rope_1"},
+                     {&g.pf_rows_qkv_rope[0][1], "pf_rows_qkv_rope_q8_1"},
+                     {&g.pf_rows_qkv_rope[1][0], "pf_rows_qkv_rope_2"},
+                     {&g.pf_rows_qkv_rope[1][1], "pf_rows_qkv_rope_q8_2"},
+                     {&g.pf_rows_qkv[0][0], "pf_rows_qkv_11"},
+                     {&g.pf_rows_qkv[0][1], "pf_rows_qkv_q8_11"},
+                     {&g.pf_rows_qkv[1][0], "pf_rows_qkv_12"},
+                     {&g.pf_rows_qkv[1][1], "pf_rows_qkv_q8_12"},
+                     {&g.pf_rows_gu[0][0], "pf_rows_gu_12"},
+                     {&g.pf_rows_gu[0][1], "pf_rows_gu_q8_12"},
+                     {&g.pf_rows_gu[1][0], "pf_rows_gu_22"},
+                     {&g.pf_rows_gu[1][1], "pf_rows_gu_q8_22"},
+                     {&g.pf_rows_gu[2][0], "pf_rows_gu_24"},
+                     {&g.pf_rows_gu[2][1], "pf_rows_gu_q8_24"},
+                     {&g.pf_rows_gu[3][0], "pf_rows_gu_26"},
+                     {&g.pf_rows_gu[3][1], "pf_rows_gu_q8_26"},
+                     {&g.pf_rows_o[0][0], "pf_rows_o_1"},
+                     {&g.pf_rows_o[0][1], "pf_rows_o_q8_1"},
+                     {&g.pf_rows_o[1][0], "pf_rows_o_2"},
+                     {&g.pf_rows_o[1][1], "pf_rows_o_q8_2"},
+                     {&g.pf_rows_dn[0][0], "pf_rows_dn_1"},
+                     {&g.pf_rows_dn[0][1], "pf_rows_dn_q8_1"},
+                     {&g.pf_rows_dn[1][0], "pf_rows_dn_2"},
+                     {&g.pf_rows_dn[1][1], "pf_rows_dn_q8_2"},
                      {&g.pf_expand, "pf_expand_q8"}};
         bool ok = true;
         for (auto& n : names) ok = ok && hipModuleGetFunction(n.fn, pm, n.name) == hipSuccess;
@@ -1774,6 +1802,42 @@ int launch_gemm_res(const void* x, int ldx, const void* wl, int K, void* y, cons
   return launch(g.pf_res_reduce, (uint32_t)(((int64_t)M * kN + 255) / 256), 256, args, st);
 }
 
+// Argument blocks of the row products (layouts shared with prefill_rows.h).
+struct RowsQkvArgs {
+  const void *h, *norm_w;
+  const void* w[3];
+  void *xn, *q, *k, *v, *q_roped, *k_cache, *v_cache;
+  const void *qn_w, *kn_w;
+  void* rope;
+  int M, start, rope_ready;
+};
+struct RowsNormArgs {
+  const void *h, *norm_w;
+  const void* w[3];
+  void *x, *y[3], *rope;
+  int M, start;
+};
+struct RowsResArgs {
+  const void *x, *w, *r;
+  void* y;
+  int M;
+};
+
+// Most tokens the row products serve: all of a layer's products, and q/k/v
+// with RoPE alone.  At 128 tokens a layer takes 39.9 us with them and 50.6
+// with the tiled GEMMs, at 160 tokens (where a workgroup's token rows are
+// normalised by twice as many workgroups as the device has CUs) 60 and 57; the
+// q/k/v one alone pays up to 256 tokens (57.0 -> 53.7 us; 300 tokens 69.5 ->
+// 72.6).
+constexpr int32_t kPfRowsMax = 128;
+constexpr int32_t kPfRowsQkvMax = 256;
+
+int launch_rows(hipFunction_t fn, int n, int tokens, int n_tiles, int threads, void* block,
+                hipStream_t st) {
+  void* args[] = {block};
+  return launch(fn, (uint32_t)((n + tokens - 1) / tokens * n_tiles), (uint32_t)threads, args, st);
+}
+
 // One layer.  xn_ready: the workspace's xn already holds rms_norm(h,
 // attn_norm of this layer) (written by the previous layer's last reduce).
 // next_norm (the next layer's attn_norm, or null): if ffn_down's reduce can
@@ -1796,14 +1860,37 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
        *attn = ws[7], *act = ws[8], *fnx = ws[9], *part = ws[10], *rope = ws[kPfRopeRegion];
   const uint32_t norm_grid = (uint32_t)((n + 15) / 16);
   int rc;
-  if (!xn_ready) {
-    void* args[] = {&h, &an, &xn, &n};
-    if ((rc = launch(g.pf_norm, norm_grid, 256, args, st))) return rc;
-  }
   // f16 layer matrices when the caller made them, else the Q8_0 stacks
   const uint8_t* f16l =
       w->prefill_f16 ? cb(w->prefill_f16) + (int64_t)layer * kPfF16Layer * 2 : nullptr;
-  if (f16l) {  // q, k, v as one [4096, 1024] matrix, output columns split three ways
+  const int q8 = f16l ? 0 : 1;
+  const bool rows = n <= kPfRowsMax, rows_qkv = n <= kPfRowsQkvMax;
+  const void* wq = f16l ? (const void*)(f16l + kPfF16Qkv * 2) : cb(w->wq) + layer * bpl_q;
+  const void* wk = cb(w->wk) + layer * bpl_kv;
+  const void* wv = cb(w->wv) + layer * bpl_kv;
+  if (n <= 64) {
+    // 16 columns a workgroup fill the CUs with one token tile; from 17 tokens
+    // on 32 columns halve the times a row is normalised (24 tokens 38.5 -> 38.2
+    // us a layer, 64 tokens 46.1 -> 44.1)
+    RowsNormArgs a{h, an, {wq, wk, wv}, xn, {q, k, v}, rope_ready ? nullptr : rope, n, p0};
+    const int i = n <= 16 ? 0 : 1;
+    if ((rc = launch_rows(g.pf_rows_qkv[i][q8], n, 16, 256 >> i, 512, &a, st))) return rc;
+  } else if (rows_qkv) {
+    // a whole head a workgroup, so RoPE and the cache writes fit behind it:
+    // 32 workgroups per token tile, enough from about 65 tokens (64 tokens
+    // 44.1 against 44.9 us a layer, 96 tokens 46.9 against 46.2)
+    RowsQkvArgs a{h, an, {wq, wk, wv}, xn, q, k, v, qr, kc, vc, qn, kn, rope, n, p0,
+                  rope_ready ? 1 : 0};
+    const int i = n <= kPfRowsMax ? 0 : 1;
+    if ((rc = launch_rows(g.pf_rows_qkv_rope[i][q8], n, 16 << i, 32, 512, &a, st))) return rc;
+  }
+  if (!rows_qkv && !xn_ready) {
+    void* args[] = {&h, &an, &xn, &n};
+    if ((rc = launch(g.pf_norm, norm_grid, 256, args, st))) return rc;
+  }
+  if (rows_qkv) {
+    // done above
+  } else if (f16l) {  // q, k, v as one [4096, 1024] matrix, output columns split three ways
     const int seg_col[2] = {2048, 3072};
     void* const y_seg[2] = {k, v};
     const int ldy_seg[2] = {1024, 1024};
@@ -1819,9 +1906,9 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
                           2048, 64, q, 2048, nullptr, 0, 0, n, st, &kv)))
       return rc;
   }
-  {
+  if (n <= 64 || !rows_qkv) {
     int start = p0;
-    if (!rope_ready) {  // the prompt positions' angles (the same for every layer)
+    if (!rope_ready && !rows_qkv) {  // the prompt positions' angles (the same for every layer)
       void* targs[] = {&start, &rope};
       if ((rc = launch(g.pf_rope_table, (uint32_t)n, 64, targs, st))) return rc;
     }
@@ -1847,6 +1934,27 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
   // split-K sums of attn_o and ffn_down
   const size_t part_bytes = pf_region_bytes(n, kPfTokenRegions);
   bool fn_done = false;
+  if (rows) {
+    // attn_o, gate/up and ffn_down as row products: 16 tokens a workgroup while
+    // that leaves CUs to fill, then 32; gate/up with 16, 16, 32 and 48 gate and
+    // up rows (each step where the next was measured faster: 32 / 64 / 128
+    // tokens)
+    const int i = n <= 64 ? 0 : 1;
+    RowsResArgs ao{attn, f16l ? (const void*)(f16l + kPfF16O * 2) : cb(w->wo) + layer * bpl_o, h,
+                   h1, n};
+    if ((rc = launch_rows(g.pf_rows_o[i][q8], n, 16 << i, 64, 512, &ao, st))) return rc;
+    RowsNormArgs gu{h1, fn,
+                    {f16l ? (const void*)(f16l + kPfF16Gu * 2) : cb(w->wgu) + layer * bpl_gu,
+                     nullptr, nullptr},
+                    fnx, {act, nullptr, nullptr}, nullptr, n, 0};
+    const int j = n <= 16 ? 0 : (n <= 32 ? 1 : (n <= 64 ? 2 : 3));
+    const int gu_tiles[4] = {192, 192, 96, 64};
+    if ((rc = launch_rows(g.pf_rows_gu[j][q8], n, j == 0 ? 16 : 32, gu_tiles[j], 512, &gu, st)))
+      return rc;
+    RowsResArgs ad{act, f16l ? (const void*)(f16l + kPfF16Dn * 2) : cb(w->wdn) + layer * bpl_dn,
+                   h1, h, n};
+    return launch_rows(g.pf_rows_dn[i][q8], n, 16 << i, 64, 768, &ad, st);
+  }
   if ((rc = launch_gemm_res(attn, 2048, cb(w->wo) + layer * bpl_o, 2048, h1, h, n, part,
                             part_bytes, st, fn, fnx, &fn_done,
                             f16l ? f16l + kPfF16O * 2 : nullptr)))
@@ -1864,6 +1972,7 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
     rc = launch_gemm(g.pf_gemm_swiglu, nullptr, fnx, 1024, cb(w->wgu) + layer * bpl_gu, 1024, 3072,
                      32, act, 3072, nullptr, 0, 3072, n, st);
   if (rc) return rc;
+  if (rows_qkv) next_norm = nullptr;  // the next layer's q/k/v product forms its norm
   return launch_gemm_res(act, 3072, cb(w->wdn) + layer * bpl_dn, 3072, h, h1, n, part, part_bytes,
                          st, next_norm, xn, next_xn_ready, f16l ? f16l + kPfF16Dn * 2 : nullptr);
 }

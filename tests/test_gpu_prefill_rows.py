@@ -1,0 +1,123 @@
+"""GPU tests of the prompt layer's row products (prefill_rows.h: all products up
+to 128 tokens, q/k/v with RoPE up to 256).
+
+Token counts sit on the edges of their 16- and 32-token tiles and of the rules
+that pick an instance.  Each product is checked against a 64-bit product of the
+GPU's own input rows and the f16 weights.  Bound: an f32 sum of K exact f16
+products is off by at most K 2^-24 sum |x w| in any order; rounding to f16 adds
+half an ulp, 2^-11 relative (2^-25 for subnormals).
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_decode import fill_cache_layer
+
+pytestmark = pytest.mark.gpu
+
+LAYER = 5
+
+
+@pytest.fixture(scope="module")
+def D():
+    from qwen3_iree_amd import decode
+
+    return decode
+
+
+@pytest.fixture(scope="module")
+def dmodel(gpu, D, model_host):
+    m = D.DeviceWeights(model_host, prefill_f16=True)
+    yield m
+    m.free()
+
+
+@pytest.fixture(scope="module")
+def w64(O, model_host):
+    w = model_host
+    return {name: O.q8_dequant_f16(m[LAYER], n, k).astype(np.float64)
+            for name, m, n, k in (("q", w.wq, 2048, 1024), ("k", w.wk, 1024, 1024),
+                                  ("v", w.wv, 1024, 1024), ("o", w.wo, 1024, 2048),
+                                  ("gu", w.wgu, 6144, 1024), ("dn", w.wdn, 1024, 3072))}
+
+
+def product(x, w):
+    """x w^T in 64 bits and the error bound of its f16 result."""
+    x = x.astype(np.float64)
+    ref = x @ w.T
+    return ref, 2.0 ** -11 * np.abs(ref) + 2.0 ** -25 + x.shape[1] * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
+
+
+def assert_within(got, ref, tol, what):
+    bad = np.argwhere(~(np.abs(got.astype(np.float64) - ref) <= tol))
+    assert bad.size == 0, (what, len(bad), bad[:4].tolist())
+
+
+def check_layer(g, h_in, w64):
+    for name in ("q", "k", "v"):
+        assert_within(g[name], *product(g["xn"], w64[name]), name)
+    for name, x, base, out in (("o", "attn", h_in, "res"), ("dn", "act", g["res"], "h")):
+        ref, tol = product(g[x], w64[name])
+        ref = base.astype(np.float64) + ref
+        assert_within(g[out], ref, tol + 2.0 ** -11 * (np.abs(ref) + tol) + 2.0 ** -25, out)
+    ref, tol = product(g["fn"], w64["gu"])
+    gate, up = ref[:, :3072], ref[:, 3072:]
+    sig = 1 / (1 + np.exp(-gate))
+    # |d silu / d gate| <= 1.1; exp, 1 + e, 1 / den, gate sig and silu up each
+    # round to f16 once: five half-ulp steps on the way to the result
+    rel = 5 * 2.0 ** -11 + 2.0 ** -10
+    want = gate * sig * up
+    assert_within(g["act"], want,
+                  1.1 * np.abs(up) * tol[:, :3072] + np.abs(gate * sig) * tol[:, 3072:]
+                  + rel * np.abs(want) + 2.0 ** -20 * (1 + np.abs(up)), "act")
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 31, 32, 33, 49, 63, 64, 65, 81, 127, 128, 129, 160,
+                               255, 256, 257])
+def test_row_products_match_f64_and_both_weight_forms_agree(gpu, D, dmodel, w64, n):
+    rng = np.random.default_rng(4100 + n)
+    p0 = 7
+    sess = D.DecodeSession(dmodel, p0 + n + 3)
+    try:
+        kc = np.zeros((28 * sess.max_seq, 1024), np.float16)
+        fill_cache_layer(sess, LAYER, p0, rng, kc, np.zeros_like(kc))
+        h_in = (1.5 * rng.standard_normal((n, 1024))).astype(np.float16)
+        res = []
+        for f16 in (True, False):
+            print(f"row products n {n} f16 {f16}", flush=True)
+            dmodel.use_prefill_matrices(f16)
+            g = sess.prefill_layer(LAYER, h_in, p0)
+            res.append((g, sess.cache_rows(LAYER, 0, sess.max_seq)))
+        (ga, ca), (gb, cb) = res
+        for name in ga:
+            assert np.array_equal(ga[name].view(np.uint16), gb[name].view(np.uint16)), name
+        for a, b in zip(ca, cb):
+            assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
+        check_layer(ga, h_in, w64)
+        assert np.array_equal(ca[1][p0:p0 + n].view(np.uint16), ga["v"].view(np.uint16))
+        assert not ca[0][p0 + n:].any() and not ca[1][p0 + n:].any()
+    finally:
+        dmodel.use_prefill_matrices(True)
+        sess.free()
+
+
+@pytest.mark.parametrize("n", [16, 100, 200])
+def test_row_products_with_the_prompts_rope_table(gpu, D, dmodel, model_host, n):
+    """qwen3_prefill_batched computes the RoPE table in its first layer and
+    reads it in the others; a layer on its own computes its angles: every
+    layer's cache rows must be the same bits."""
+    prompt = np.random.default_rng(4200 + n).integers(0, D.VOCAB, n).astype(np.int32)
+    print(f"row products rope table n {n}", flush=True)
+    a, b = D.DecodeSession(dmodel, n + 1), D.DecodeSession(dmodel, n + 1)
+    try:
+        a.set_state(0, 0)
+        a.prefill_batched(prompt)
+        h = model_host.token_embd[prompt]
+        for layer in range(28):
+            h = b.prefill_layer(layer, h, 0)["h"]
+            for x, y in zip(a.cache_rows(layer, 0, n), b.cache_rows(layer, 0, n)):
+                assert np.array_equal(x.view(np.uint16), y.view(np.uint16)), layer
+    finally:
+        a.free()
+        b.free()
