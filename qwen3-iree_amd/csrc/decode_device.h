@@ -16,9 +16,16 @@ constexpr int kKvHeads = 8;
 constexpr int kQHeads = 16;
 constexpr int kFfn = 3072;
 constexpr int kVocab = 151936;
-constexpr int kAttnSplits = 32;      // position splits per kv head (one wave each)
+// Position splits per kv head (one wave each): 32 up to a context of
+// kAttnShortCtx, where a split is at most two chunks of 32 positions; 64 above, where
+// the attention is bound by the bytes the waves have in flight (32 splits: 256
+// waves x 16 KiB, 1.63 us per chunk and wave, 2.6 TB/s).  Single-launch step
+// with 32 / 64 splits, context 2048 / 4096 / 8192 / 16384: LONG_FIGURES.
+constexpr int kAttnSplits = 32;
+constexpr int kAttnShortCtx = 2048;
 constexpr int kAttnWaves = 4;        // splits per workgroup, merged in LDS
 constexpr int kAttnGroups = kAttnSplits / kAttnWaves;  // partials per query head
+constexpr int kAttnGroupsMax = 2 * kAttnGroups;
 constexpr int kPartStride = 4 + kHeadDim;  // m, l, 2 pad, acc[128] (16-byte aligned acc)
 constexpr float kEps = 9.99999997e-7f;    // qwen3_full.mlir:63
 constexpr float kRopeBase = 1.0e6f;       // qwen3_full.mlir:59
@@ -267,28 +274,28 @@ __device__ __forceinline__ uint16_t residual_f16(_Float16 base, float acc) {
   return __builtin_bit_cast(uint16_t, (_Float16)(base + to_f16(acc)));
 }
 
-// Weights of the 8 split-group partials of one query head: w_g = 2^(m_g -
+// Weights of the N split-group partials of one query head: w_g = 2^(m_g -
 // max m) (the maxima are in base-2 units; 0 for an empty group), L = sum_g l_g w_g, summed in group order.
-__device__ __forceinline__ void merge_weights(const float (&m)[kAttnGroups],
-                                              const float (&l)[kAttnGroups],
-                                              float (&w)[kAttnGroups], float& L) {
+template <int N>
+__device__ __forceinline__ void merge_weights(const float (&m)[N], const float (&l)[N],
+                                              float (&w)[N], float& L) {
   float M = -__builtin_inff();
 #pragma unroll
-  for (int g = 0; g < kAttnGroups; ++g) M = fmaxf(M, m[g]);
+  for (int g = 0; g < N; ++g) M = fmaxf(M, m[g]);
   L = 0.0f;
 #pragma unroll
-  for (int g = 0; g < kAttnGroups; ++g) {
+  for (int g = 0; g < N; ++g) {
     w[g] = m[g] == -__builtin_inff() ? 0.0f : exp2f(m[g] - M);
     L = L + l[g] * w[g];
   }
 }
 
 // One merged output dim: sum_g acc_g w_g in group order.
-__device__ __forceinline__ float merge_dim(const float (&acc)[kAttnGroups],
-                                           const float (&w)[kAttnGroups]) {
+template <int N>
+__device__ __forceinline__ float merge_dim(const float (&acc)[N], const float (&w)[N]) {
   float a = 0.0f;
 #pragma unroll
-  for (int g = 0; g < kAttnGroups; ++g) a = a + acc[g] * w[g];
+  for (int g = 0; g < N; ++g) a = a + acc[g] * w[g];
   return a;
 }
 
@@ -310,16 +317,28 @@ __device__ __forceinline__ void rope_angles(int pos, float (&cs)[2], float (&sn)
   for (int dd = 0; dd < 2; ++dd) rope_angle(pos, (2 * lane + dd) & 63, cs[dd], sn[dd]);
 }
 
-// Position range [start, end) of attention split s (of kAttnSplits) over ctx
-// = pos + 1 positions, and the last row a clamped load may touch.
+// log2 of the number of splits of the attention at (clamped) position pos.
+__device__ __forceinline__ int attn_splits_log2(int pos) {
+  static_assert(kAttnSplits == 32, "log2");
+  return pos < kAttnShortCtx ? 5 : 6;
+}
+__device__ __forceinline__ int attn_splits(int pos) { return 1 << attn_splits_log2(pos); }
+// Its chunks of 32 positions per split (the most any split has).
+__device__ __forceinline__ int attn_chunks(int pos) {
+  const int lg = attn_splits_log2(pos);
+  return (((pos + (1 << lg)) >> lg) + 31) / 32;
+}
+
+// Position range [start, end) of attention split s over ctx = pos + 1
+// positions, and the last row a clamped load may touch.
 struct SplitRange {
   int start, end, last;
 };
 __device__ __forceinline__ SplitRange split_range(int s, int pos) {
-  const int ctx = pos + 1;
+  const int ctx = pos + 1, lg = attn_splits_log2(pos);
   SplitRange r;
-  r.start = (int)((int64_t)s * ctx / kAttnSplits);
-  r.end = (int)((int64_t)(s + 1) * ctx / kAttnSplits);
+  r.start = (int)(((int64_t)s * ctx) >> lg);
+  r.end = (int)(((int64_t)(s + 1) * ctx) >> lg);
   r.last = r.end - 1 > 0 ? r.end - 1 : 0;
   return r;
 }
@@ -422,7 +441,7 @@ struct __attribute__((aligned(16))) AttnLds {
 };
 
 // Attention for kv head g and split group sg: four waves, wave w taking
-// position split s = 4 sg + w of the 32 equal splits of ctx = pos + 1; the
+// position split s = 4 sg + w of the equal splits of ctx = pos + 1; the
 // four results merge in LDS into one partial per query head and group.  Per
 // wave:
 //  0. the split's cache rows go through the wave's LDS region kv
@@ -476,14 +495,13 @@ __device__ __forceinline__ void attention_group(AttnLds& L, int g, int sg, int p
   nwv[1] = nwv[0];
 
   const int pos = pos_raw < 0 ? 0 : (pos_raw >= max_seq ? max_seq - 1 : pos_raw);
-  const int ctx = pos + 1;
   const SplitRange sr = split_range(s, pos);
   const int start = sr.start;
   const int end = sr.end;
   // this workgroup's four splits hold position pos: it writes the new k / v
   const bool owns_pos = split_range(sg * kAttnWaves, pos).start <= pos &&
                         pos < split_range(sg * kAttnWaves + kAttnWaves - 1, pos).end;
-  const int n_chunks = ((ctx + kAttnSplits - 1) / kAttnSplits + 31) / 32;  // workgroup-uniform
+  const int n_chunks = attn_chunks(pos);  // workgroup-uniform
 
   // ---- 0. first chunk of the cache (rows clamped into [start, end - 1],
   // row 0 for an empty split), staged into this wave's LDS region unless the

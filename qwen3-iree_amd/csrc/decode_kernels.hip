@@ -16,7 +16,7 @@
 // plus dec_embed (token row gather), dec_vocab_argmax (final rms_norm fused
 // into the vocab GEMV + argmax) and dec_finalize (token, position).
 //
-// Single launch: dec_step runs the whole step in one launch of 448
+// Single launch: dec_step runs the whole step in one launch of 512
 // workgroups, two per CU and all resident at once, phases handing activations
 // over through tagged 8-byte words instead of kernel boundaries (see its
 // comment).
@@ -24,6 +24,8 @@
 // Numerics follow the reference op by op: f16 tensors between ops, f32 in
 // reductions and transcendental math, RNE to f16.  Normalisation multiplies by
 // 1/rms where the reference divides by rms (one f32 rounding apart).
+#include <type_traits>
+
 #include "decode_device.h"
 
 // ------------------------------------------------------------- kernels ----
@@ -73,9 +75,10 @@ extern "C" __global__ __launch_bounds__(64) void dec_qkv(
       [&](int row, float acc) { y[row] = f32_to_f16_bits(acc); });
 }
 
-// Attention for kv head g = block / 8 and split group sg = block % 8 (see
+// Attention for kv head g = (block / 8) mod 8 and split group sg = block % 8,
+// + 8 for blocks from 64 on, which only a context of 64 splits has (see
 // attention_group): q/k/v from global memory, the partial (m, l, acc[128]) of
-// each query head to part[head][sg] (the attn_o kernel merges the 8 groups).
+// each query head to part[head][sg] (the attn_o kernel merges the groups).
 extern "C" __global__ __launch_bounds__(256) void dec_attention(
     const uint16_t* __restrict__ q_raw, const uint16_t* __restrict__ k_raw,
     const uint16_t* __restrict__ v_raw, const uint16_t* __restrict__ qn_w,
@@ -84,12 +87,14 @@ extern "C" __global__ __launch_bounds__(256) void dec_attention(
     uint16_t* __restrict__ q_roped) {
   __shared__ AttnLds lds;
   __shared__ __attribute__((aligned(16))) uint8_t kv[kAttnWaves][kKvPrefetchBytes];
-  const int g = blockIdx.x / kAttnGroups;
-  const int sg = blockIdx.x % kAttnGroups;
+  const int g = blockIdx.x / kAttnGroups % kKvHeads;
+  const int sg = blockIdx.x % kAttnGroups + blockIdx.x / (kAttnGroups * kKvHeads) * kAttnGroups;
   const int lane = threadIdx.x & 63;
   const int pos_raw = *pos_ptr;
+  const int pos = pos_raw < 0 ? 0 : (pos_raw >= max_seq ? max_seq - 1 : pos_raw);
+  if (kAttnWaves * sg >= attn_splits(pos)) return;
   float cs[2], sn[2];
-  rope_angles(pos_raw < 0 ? 0 : (pos_raw >= max_seq ? max_seq - 1 : pos_raw), cs, sn);
+  rope_angles(pos, cs, sn);
   attention_group(
       lds, g, sg, pos_raw, cs, sn, max_seq, qn_w, kn_w, k_cache, v_cache, q_roped,
       kv[threadIdx.x >> 6], false, [] {},
@@ -100,7 +105,7 @@ extern "C" __global__ __launch_bounds__(256) void dec_attention(
         v_new = load_global(reinterpret_cast<const uint32_t*>(v_raw + g * kHeadDim) + lane);
       },
       [&](int hh, float M, float L, float a0, float a1) {
-        float* dst = part + ((size_t)(2 * g + hh) * kAttnGroups + sg) * kPartStride;
+        float* dst = part + ((size_t)(2 * g + hh) * kAttnGroupsMax + sg) * kPartStride;
         if (lane == 0) {
           dst[0] = M;
           dst[1] = L;
@@ -109,64 +114,91 @@ extern "C" __global__ __launch_bounds__(256) void dec_attention(
       });
 }
 
+// The partials of one query head's 8 dims d0 .. from ph, groups G0 .. G0 + 7.
+struct Partials {
+  float2 ml[kAttnGroupsMax];
+  u32x4 av[kAttnGroupsMax][2];
+};
+template <int G0>
+__device__ __forceinline__ void load_partials(Partials& p, const float* __restrict__ ph, int d0) {
+#pragma unroll
+  for (int gi = G0; gi < G0 + kAttnGroups; ++gi) {
+    const float* pg = ph + (size_t)gi * kPartStride;
+    p.ml[gi] = *reinterpret_cast<const float2*>(pg);
+    p.av[gi][0] = load_global(reinterpret_cast<const u32x4*>(pg + 4 + d0));
+    p.av[gi][1] = load_global(reinterpret_cast<const u32x4*>(pg + 4 + d0) + 1);
+  }
+}
+// The first N of them merged, as four f16 pairs.
+template <int N>
+__device__ __forceinline__ u32x4 merge_partials(const Partials& p) {
+  float mg[N], lg[N], wg[N], L;
+#pragma unroll
+  for (int gi = 0; gi < N; ++gi) {
+    mg[gi] = p.ml[gi].x;
+    lg[gi] = p.ml[gi].y;
+  }
+  merge_weights(mg, lg, wg, L);
+  float a[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    // copy the elements out first: __builtin_bit_cast of a vector
+    // element lvalue reads element 0 with this compiler
+    float accg[N];
+#pragma unroll
+    for (int gi = 0; gi < N; ++gi) {
+      const uint32_t bits = p.av[gi][e >> 2][e & 3];
+      accg[gi] = __builtin_bit_cast(float, bits);
+    }
+    a[e] = merge_dim(accg, wg);
+  }
+  return (u32x4){pack_f16x2(a[0] / L, a[1] / L), pack_f16x2(a[2] / L, a[3] / L),
+                 pack_f16x2(a[4] / L, a[5] / L), pack_f16x2(a[6] / L, a[7] / L)};
+}
+
 // attn = the merged attention output: head h, dim d =
-// sum_g w_g acc_g[d] / sum_g w_g l_g over the 8 partials g of head h, w_g =
-// 2^(m_g - max m) (m in base-2 units); then res = h + f16(W_o[layer] . attn)
-// (qwen3_full.mlir:739, 801-805).  Four waves per workgroup, one row quad
-// each; the workgroup's 256 threads merge 8 dims each into LDS while the
-// weight loads are in flight.  Workgroup 0 also stores attn.
+// sum_g w_g acc_g[d] / sum_g w_g l_g over the partials g of head h (8, or 16
+// at a context of 64 splits), w_g = 2^(m_g - max m) (m in base-2 units); then
+// res = h + f16(W_o[layer] . attn) (qwen3_full.mlir:739, 801-805).  Four waves
+// per workgroup, one row quad each; the workgroup's 256 threads merge 8 dims
+// each into LDS while the weight loads are in flight.  Workgroup 0 also stores
+// attn.
 extern "C" __global__ __launch_bounds__(256) void dec_o_res(const uint8_t* __restrict__ wo,
                                                             const float* __restrict__ part,
                                                             const uint16_t* __restrict__ h,
                                                             uint16_t* __restrict__ res,
-                                                            uint16_t* __restrict__ attn_out) {
+                                                            uint16_t* __restrict__ attn_out,
+                                                            const int32_t* __restrict__ pos_ptr,
+                                                            int max_seq) {
   constexpr int LDSB = QuadShape<2>::LDS_BYTES;
   __shared__ __attribute__((aligned(16))) uint8_t lds[4 * LDSB];
   __shared__ __attribute__((aligned(16))) uint16_t attn[2 * kHidden];
   const int t = threadIdx.x;
   const int wave = t >> 6;
+  const int pos_raw = *pos_ptr;
   // the residual of this lane's row, requested up front; all 1024 rows exist,
   // and every lane of a row group stores the (same) result, so nothing here
   // is conditional and the load stays ahead of the GEMV
   const int row = 4 * (4 * blockIdx.x + wave) + ((t & 63) >> 4);
   const _Float16 h_row = as_half(load_global_u16(h + row));
+  // the partials every context has, ahead of the weights: they return first
+  // and are merged while the weights are in flight
+  const float* ph = part + (size_t)(t >> 4) * kAttnGroupsMax * kPartStride;
+  const int d0 = 8 * (t & 15);
+  Partials p;
+  load_partials<0>(p, ph, d0);
+  __builtin_amdgcn_sched_barrier(0);
   const float acc = q8_quad_core_acc<2>(
       wo, kHidden, 4 * blockIdx.x + wave, lds + wave * LDSB,
       [&](u32x4 (&xr)[2][8]) {
-        const int head = t >> 4;
-        const int d0 = 8 * (t & 15);
-        const float* ph = part + (size_t)head * kAttnGroups * kPartStride;
-        float2 ml[kAttnGroups];
-        u32x4 av[kAttnGroups][2];
-#pragma unroll
-        for (int gi = 0; gi < kAttnGroups; ++gi) {
-          const float* pg = ph + (size_t)gi * kPartStride;
-          ml[gi] = *reinterpret_cast<const float2*>(pg);
-          av[gi][0] = load_global(reinterpret_cast<const u32x4*>(pg + 4 + d0));
-          av[gi][1] = load_global(reinterpret_cast<const u32x4*>(pg + 4 + d0) + 1);
+        const int pos = pos_raw < max_seq ? pos_raw : max_seq - 1;
+        u32x4 packed;
+        if (attn_splits(pos) == kAttnSplits) {
+          packed = merge_partials<kAttnGroups>(p);
+        } else {
+          load_partials<kAttnGroups>(p, ph, d0);
+          packed = merge_partials<kAttnGroupsMax>(p);
         }
-        float mg[kAttnGroups], lg[kAttnGroups], wg[kAttnGroups], L;
-#pragma unroll
-        for (int gi = 0; gi < kAttnGroups; ++gi) {
-          mg[gi] = ml[gi].x;
-          lg[gi] = ml[gi].y;
-        }
-        merge_weights(mg, lg, wg, L);
-        float a[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          // copy the elements out first: __builtin_bit_cast of a vector
-          // element lvalue reads element 0 with this compiler
-          float accg[kAttnGroups];
-#pragma unroll
-          for (int gi = 0; gi < kAttnGroups; ++gi) {
-            const uint32_t bits = av[gi][e >> 2][e & 3];
-            accg[gi] = __builtin_bit_cast(float, bits);
-          }
-          a[e] = merge_dim(accg, wg);
-        }
-        const u32x4 packed = {pack_f16x2(a[0] / L, a[1] / L), pack_f16x2(a[2] / L, a[3] / L),
-                              pack_f16x2(a[4] / L, a[5] / L), pack_f16x2(a[6] / L, a[7] / L)};
         reinterpret_cast<u32x4*>(attn)[t] = packed;
         if (blockIdx.x == 0) reinterpret_cast<u32x4*>(attn_out)[t] = packed;
         __syncthreads();
@@ -279,8 +311,9 @@ extern "C" __global__ __launch_bounds__(256) void dec_scratch_clear(uint32_t* __
 
 // ======================================================= single launch ====
 //
-// dec_step: the whole decode step in one launch of kStepWgs = 448 workgroups
-// x 256 threads, two per CU, all resident at once (the launcher checks the
+// dec_step: the whole decode step in one launch of kStepGrid = 512 workgroups
+// x 256 threads (448 of them with a role unless the context is long), two per
+// CU, all resident at once (the launcher checks the
 // occupancy; there is no grid barrier, and every wait is bounded).  Work
 // moves between workgroups as tagged words: a 64-bit word holds 32 bits of
 // data (an f16 pair or an f32) and a 32-bit tag naming (step, layer, phase); a
@@ -305,6 +338,9 @@ extern "C" __global__ __launch_bounds__(256) void dec_scratch_clear(uint32_t* __
 //                 merges its kv head's 8 partials of both query heads -> ATT
 //                 words; then the next layer's first cache chunk is requested
 //                 into LDS.
+//       448..511  the same for split groups 8 .. 15 of a long context (64
+//                 splits, see kAttnShortCtx), where split groups 0 and 1 merge
+//                 one query head each; at other contexts they end at once
 //   CE  320..447  C: attn_o + residual, row quads 2 c, 2 c + 1 (c = wg - 320),
 //                 one 1024-column chunk per wave, summed in LDS -> RES words;
 //                 then E: ffn_down + residual over the same two row quads,
@@ -321,6 +357,9 @@ extern "C" __global__ __launch_bounds__(256) void dec_scratch_clear(uint32_t* __
 namespace {
 
 constexpr int kStepWgs = 448;
+// The launch: 64 more workgroups (the second slot of the remaining CUs), which
+// take split groups 8 .. 15 of a context of 64 splits and end at once below.
+constexpr int kStepGrid = 512;
 constexpr int kAdBase = 0, kDCount = 192;  // A on all 256, D on the first 192
 constexpr int kBBase = 256;                // 64 attention workgroups
 constexpr int kCBase = 320;                // 128 attn_o + ffn_down workgroups
@@ -355,7 +394,7 @@ constexpr int kWQ = kWH + kRep * kNH;                      // 1024: q row pairs
 constexpr int kWK = kWQ + 1024;                            // 512
 constexpr int kWV = kWK + 512;                             // 512
 constexpr int kWPart = kWV + 512;                          // 16 x 8 x 130
-constexpr int kWAtt = kWPart + kQHeads * kAttnGroups * 130;  // kRep x 1024
+constexpr int kWAtt = kWPart + kQHeads * kAttnGroupsMax * 130;  // kRep x 1024
 constexpr int kWRes = kWAtt + kRep * kNAtt;                // kRep x 512
 constexpr int kWAct = kWRes + kRep * kNRes;                // kRep x 1536
 constexpr int kWParity = kWAct + kRep * kNAct;
@@ -589,7 +628,7 @@ __device__ __forceinline__ int stamp_slot(int wg) {
   return -1;
 }
 
-constexpr int kVecWords = 2 * kAttnGroups * 130;  // 2080: the largest polled vector
+constexpr int kVecWords = kAttnGroupsMax * 130;  // 2080: the largest polled vector
 // Weight prefetches sleep 64 kPace* cycles between 1 KiB pieces, each set
 // spread over the time its role has before the weights are needed (the gate/up
 // weights are requested right after A, the next q/k/v weights right after D,
@@ -606,8 +645,13 @@ constexpr int kVecWords = 2 * kAttnGroups * 130;  // 2080: the largest polled ve
 // kernel arguments preloaded (508.5 / 511.4 as below): D 26 / 34 526.8 /
 // 542.6, A 28 / 36 515.1 / 524.4, C 26 / 34 515.3 / 529.5, E 12 / 20 512.2 /
 // 510.9.
+// With split groups 8 .. 15 in the code (context 1024 / 16384): A 28 / 30 / 32
+// / 34 519 / 513 / 516 / 522 and 1016 / 1011 / 1008 / 1006, so A sleeps 30 where
+// a split is one chunk and 32 where the attention takes longer (2048: 592 at 30,
+// PACE2048 at 32); C 28 / 32 517-519, D 28 / 32 521 / 530, E 12 / 20 and the
+// cache chunk 4 / 12 within 1.
 #ifndef DEC_PACE_A
-#define DEC_PACE_A 32
+#define DEC_PACE_A 30
 #endif
 #ifndef DEC_PACE_D
 #define DEC_PACE_D 30
@@ -655,6 +699,9 @@ static_assert(kVocabWgs > 256 || kVocabHeavy16 == 16,
 static_assert(kVocab / 4 * 16 / (4 * (256 * kVocabHeavy16 + (kVocabWgs - 256) * 16)) - 1 >=
                   kVocabPre + 2,
               "vocab batches per wave");
+static_assert(kStepGrid - kStepWgs == kKvHeads * (kAttnGroupsMax - kAttnGroups) &&
+                  kStepWgs % 8 == 0 && (kStepWgs - kBBase) % kKvHeads == 0,
+              "the further split groups, one kv head per XCD (wg mod 8)");
 static_assert(kKvHeads == 8 && kBBase % 8 == 0, "one kv head's attention workgroups per XCD (wg mod 8)");
 
 }  // namespace
@@ -701,19 +748,21 @@ void dec_step(StepParams P) {
     give_up(P.status, P.seq, seq);  // the host forces a give-up
     s_abort = 1;
   }
-  // Workgroups start in index order: the last one marks the launch as
+  const int pos_raw = *P.pos;
+  const int pos_c = pos_raw < 0 ? 0 : (pos_raw >= P.max_seq ? P.max_seq - 1 : pos_raw);
+  const bool long_ctx = attn_splits(pos_c) != kAttnSplits;
+  // Workgroups start in index order: the last one of those every context needs
+  // marks the launch as
   // resident (a wait that finds another number after ~1 ms knows the grid
   // is not resident at once).
   if (wg == kStepWgs - 1 && t == 0)
     __hip_atomic_store(P.last_started, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int pos_raw = *P.pos;
   int tok = *P.token_in;
   tok = (tok < 0 || tok >= kVocab) ? 0 : tok;
   const uint16_t* emb = P.token_embd + (size_t)tok * kHidden;
   const Waiter W{P.last_started, P.status, P.seq, seq, P.spin_limit, &s_abort};
-  const int pos_c = pos_raw < 0 ? 0 : (pos_raw >= P.max_seq ? P.max_seq - 1 : pos_raw);
   __syncthreads();
-  if (s_abort) return;
+  if (s_abort || (wg >= kStepWgs && !long_ctx)) return;
 
   if (wg < kBBase) {
     // ================= AD: q/k/v of every layer; gate/up on 0..191 =================
@@ -729,7 +778,8 @@ void dec_step(StepParams P) {
     // kv_touch task of this wave: head wg mod 8, task (wg / 8) * 4 + wave of
     // that head's 128 = split (task mod 32), chunk 1 + task / 32 (1-4)
     const int touch_task = (wg >> 3) * 4 + wave;
-    const int n_split_chunks = ((pos_c + 1 + kAttnSplits - 1) / kAttnSplits + 31) / 32;
+    const int n_split_chunks = attn_chunks(pos_c);
+    const int splits_log2 = attn_splits_log2(pos_c), n_splits = 1 << splits_log2;
     uint8_t* const lg = S.ad.wd[wave][0];
     uint8_t* const lu = S.ad.wd[wave][1];
     q8_quad_prefetch<1>(wsel, n, qd, la);
@@ -769,11 +819,11 @@ void dec_step(StepParams P) {
       // 1158.6 -> 1094.6, 16384 1763.7 -> 1714.0, 1024 unchanged.  Touching
       // the later chunks too (two tasks per wave) measured slower (8192:
       // 1123.0, 16384: 1749.1): L2 holds only so much beside the weights.
-      if (touch_task < 32 * (n_split_chunks - 1)) {
-        const SplitRange tr = split_range(touch_task & 31, pos_c);
+      if (touch_task < n_splits * (n_split_chunks - 1)) {
+        const SplitRange tr = split_range(touch_task & (n_splits - 1), pos_c);
         kv_touch(S.ad.sink[wave], P.k_cache + (int64_t)layer * P.max_seq * (kKvHeads * kHeadDim),
                  P.v_cache + (int64_t)layer * P.max_seq * (kKvHeads * kHeadDim), wg & 7,
-                 tr.start + 32 * (1 + (touch_task >> 5)), tr.last);
+                 tr.start + 32 * (1 + (touch_task >> splits_log2)), tr.last);
       }
       // The A-only workgroups (idle until the next layer's h) bring the
       // gate/up quads of the 24 D workgroups on their XCD (wg mod 8) into its
@@ -821,16 +871,20 @@ void dec_step(StepParams P) {
                    step_tag(seq, layer, kPhAct));
         STAMP(layer, 10);
       }
-      if (layer + 1 < kLayers) q8_quad_prefetch<1, kPaceA>(wsel + (layer + 1) * bpl, n, qd, la);
+      if (layer + 1 < kLayers) {
+        if (n_split_chunks == 1) q8_quad_prefetch<1, kPaceA>(wsel + (layer + 1) * bpl, n, qd, la);
+        else q8_quad_prefetch<1, kPaceA + 2>(wsel + (layer + 1) * bpl, n, qd, la);
+      }
     }
-  } else if (wg < kCBase) {
+  } else if (wg < kCBase || wg >= kStepWgs) {
     // ================= B: attention (+ merge on split group 0) =================
     // kv head g's split groups, its merge (split group 0) among them, on
     // workgroups wg = g (mod 8): the partials' hand-off stays within one XCD
     // (one L2)
     const int bw = wg - kBBase;
     const int g = bw % kKvHeads;
-    const int sg = bw / kKvHeads;
+    const int sg = wg < kStepWgs ? bw / kKvHeads : kAttnGroups + (wg - kStepWgs) / kKvHeads;
+    const int groups = long_ctx ? kAttnGroupsMax : kAttnGroups;
     uint8_t* const kv_mine = S.b.kv[wave];
     // the first chunk of each wave's split stays in LDS: requested for layer 0
     // now, for layer l + 1 as soon as layer l's attention (and merge) is done
@@ -863,7 +917,7 @@ void dec_step(StepParams P) {
             v_new = vec[192 + lane];
           },
           [&](int hh, float M, float Ls, float a0, float a1) {
-            uint64_t* d = cur + kWPart + ((2 * g + hh) * kAttnGroups + sg) * 130;
+            uint64_t* d = cur + kWPart + ((2 * g + hh) * groups + sg) * 130;
             const uint32_t tp = step_tag(seq, layer, kPhPart);
             if (lane == 0) {
               put_word(d, __builtin_bit_cast(uint32_t, M), tp);
@@ -888,35 +942,44 @@ void dec_step(StepParams P) {
         return;
       }
       STAMP(layer, 4);
-      if (sg == 0) {
-        // the 8 groups' partials of query heads 2g, 2g+1 (contiguous words)
-        if (!W.wait(cur + kWPart + 2 * g * kAttnGroups * 130, 2 * kAttnGroups * 130,
-                    step_tag(seq, layer, kPhPart), vec))
+      // Query head qh's N partials, in vec from word v0 on, merged: this lane's
+      // two dims -> ATT words.
+      auto merge_head = [&](auto n, int qh, int v0) {
+        constexpr int N = decltype(n)::value;
+        const float* pv = reinterpret_cast<const float*>(vec) + v0;
+        float mg[N], lg[N], wgt[N], Ls;
+#pragma unroll
+        for (int gi = 0; gi < N; ++gi) {
+          mg[gi] = pv[gi * 130];
+          lg[gi] = pv[gi * 130 + 1];
+        }
+        merge_weights(mg, lg, wgt, Ls);
+        float a[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float accg[N];
+#pragma unroll
+          for (int gi = 0; gi < N; ++gi) accg[gi] = pv[gi * 130 + 2 + 2 * lane + e];
+          a[e] = merge_dim(accg, wgt);
+        }
+        const uint32_t att = pack_f16x2(a[0] / Ls, a[1] / Ls);
+#pragma unroll
+        for (int r = 0; r < kRep; ++r)
+          put_word(cur + kWAtt + r * kNAtt + qh * 64 + lane, att, step_tag(seq, layer, kPhAtt));
+      };
+      // 8 groups: split group 0 merges both heads; 16: groups 0 and 1 one each
+      // (2080 contiguous words either way)
+      if (sg < (long_ctx ? 2 : 1)) {
+        if (!W.wait(cur + kWPart + (2 * g * groups + sg * kAttnGroupsMax) * 130,
+                    kAttnGroupsMax * 130, step_tag(seq, layer, kPhPart), vec))
           return;
         STAMP(layer, 5);
-        if (wave < 2) {
-          const int hh = wave;
-          const float* pv = reinterpret_cast<const float*>(vec) + hh * kAttnGroups * 130;
-          float mg[kAttnGroups], lg[kAttnGroups], wgt[kAttnGroups], Ls;
-#pragma unroll
-          for (int gi = 0; gi < kAttnGroups; ++gi) {
-            mg[gi] = pv[gi * 130];
-            lg[gi] = pv[gi * 130 + 1];
-          }
-          merge_weights(mg, lg, wgt, Ls);
-          float a[2];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            float accg[kAttnGroups];
-#pragma unroll
-            for (int gi = 0; gi < kAttnGroups; ++gi) accg[gi] = pv[gi * 130 + 2 + 2 * lane + e];
-            a[e] = merge_dim(accg, wgt);
-          }
-          const uint32_t att = pack_f16x2(a[0] / Ls, a[1] / Ls);
-#pragma unroll
-          for (int r = 0; r < kRep; ++r)
-            put_word(cur + kWAtt + r * kNAtt + (2 * g + hh) * 64 + lane, att,
-                     step_tag(seq, layer, kPhAtt));
+        if (long_ctx) {
+          if (wave == 0)
+            merge_head(std::integral_constant<int, kAttnGroupsMax>{}, 2 * g + sg, 0);
+        } else if (wave < 2) {
+          merge_head(std::integral_constant<int, kAttnGroups>{}, 2 * g + wave,
+                     wave * kAttnGroups * 130);
         }
         STAMP(layer, 6);
         __syncthreads();  // vec is reused by the next wait

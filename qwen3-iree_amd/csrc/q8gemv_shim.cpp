@@ -49,7 +49,8 @@ constexpr KindInfo kKinds[5] = {
 };
 
 constexpr int kVocabMaxWorkgroups = 8192;
-constexpr int kStepWorkgroups = 448;  // dec_step's fixed grid (up to two workgroups per CU)
+constexpr int kStepWorkgroups = 448;  // dec_step's workgroups with a role at any context
+constexpr int kStepGrid = 512;        // its launch: two workgroups per CU (long contexts)
 constexpr uint32_t kDefaultSpinLimit = 1u << 20;  // dec_step: poll rounds before a wait gives up
 constexpr int kQ8MaxWorkgroups = 65536;
 constexpr int64_t kBatchWavesPerCu = 10;  // q8gemv_batch default
@@ -430,7 +431,7 @@ int q8gemv_init(const char* code_object_path) {
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
-  // The single-launch step needs its 448 workgroups resident together (they
+  // The single-launch step needs its 512 workgroups resident together (they
   // wait on each other's tagged words; there is no grid barrier): a device
   // whose CUs hold them all at once (two per CU), checked from the kernel's
   // occupancy.  It is launched as an ordinary kernel: a cooperative launch
@@ -444,7 +445,7 @@ int q8gemv_init(const char* code_object_path) {
     int per_cu = 0;
     if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, g.dec_step, 256, 0) ==
         hipSuccess)
-      g.step_capable = per_cu >= 1 && (int64_t)per_cu * cus >= kStepWorkgroups;
+      g.step_capable = per_cu >= 1 && (int64_t)per_cu * cus >= kStepGrid;
   }
   // The single launch is the default where it can run: no kernel boundaries,
   // and every workgroup requests its next weights before it waits.
@@ -1209,7 +1210,8 @@ constexpr int kLayers = 28;
 constexpr int kVocabRows = 151936;
 constexpr int64_t kKvRow = 8 * 128;  // f16 elements per cache slot
 constexpr int kKvHeads = 8;
-constexpr int kAttnGroupsHost = 8;  // attention workgroups (partials) per kv head
+// attention workgroups (partials) per kv head at most: 16 above 2048 positions, else 8
+constexpr int kAttnGroupsHost = 16;
 constexpr int32_t kGenerateBatch = 4;  // tokens between EOS checks (qwen3_full.mlir:1412)
 
 
@@ -1228,14 +1230,14 @@ constexpr size_t kScrXn = kScrAct + 6144;    // f16[1024] rms_norm(h, attn_norm)
 constexpr size_t kScrQr = kScrXn + 2048;     // f16[2048] q after head norm + RoPE
 constexpr size_t kScrFn = kScrQr + 4096;     // f16[1024] rms_norm(res, ffn_norm)
 constexpr size_t kScrOn = kScrFn + 2048;     // f16[1024] rms_norm(h, output_norm)
-constexpr size_t kScrPart = kScrOn + 2048;   // f32[16][8][132] attention partials
+constexpr size_t kScrPart = kScrOn + 2048;   // f32[16][16][132] attention partials
 constexpr size_t kScrSeq = 16;       // u32 step sequence number (single-launch step)
 constexpr size_t kScrStarted = 128;  // u32 the last launch whose grid was resident
 // tagged words of the single-launch step (u64; map in decode_kernels.hip)
 // the single-launch step's tagged words per layer parity: h, attention output,
 // attn_o + residual output and SwiGLU output in 4 replicas each, q/k/v and
 // the attention partials once (layout in decode_kernels.hip)
-constexpr size_t kStepWordsParity = 4 * 512 + 1024 + 512 + 512 + 16 * 8 * 130 + 4 * 1024 +
+constexpr size_t kStepWordsParity = 4 * 512 + 1024 + 512 + 512 + 16 * 16 * 130 + 4 * 1024 +
                                     4 * 512 + 4 * 1536;
 constexpr size_t kStepWords = 2 * kStepWordsParity + 2 * kStepWorkgroups;
 constexpr size_t kScrWords = (kScrPart + 16 * kAttnGroupsHost * 132 * 4 + 255) / 256 * 256;
@@ -1322,7 +1324,7 @@ int launch_step(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cs));
   if (cs != hipStreamCaptureStatusNone) {
-    hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepWorkgroups, 1, 1, 256, 1, 1, 0, st,
+    hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepGrid, 1, 1, 256, 1, 1, 0, st,
                                          args, nullptr);
     if (e != hipSuccess) return hip_fail(e, "launch of dec_step");
     return Q8_OK;
@@ -1335,7 +1337,7 @@ int launch_step(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
     HIP_TRY(hipEventCreateWithFlags(&g.step_ev, hipEventDisableTiming | hipEventDisableSystemFence));
   else if (g.step_last != st)
     HIP_TRY(hipStreamWaitEvent(st, g.step_ev, 0));
-  hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepWorkgroups, 1, 1, 256, 1, 1, 0, st, args,
+  hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepGrid, 1, 1, 256, 1, 1, 0, st, args,
                                        nullptr);
   if (e != hipSuccess) return hip_fail(e, "launch of dec_step");
   HIP_TRY(hipEventRecord(g.step_ev, st));
@@ -1458,7 +1460,8 @@ int launch_layer(const qwen3_weights* w, int layer, void* k_cache, void* v_cache
     if ((rc = launch(g.dec_attn, 8 * kAttnGroupsHost, 256, args, st))) return rc;
   }
   {
-    void* args[] = {&wo, &part, &hin, &res, &attn};
+    const void* pp = pos;
+    void* args[] = {&wo, &part, &hin, &res, &attn, &pp, &ms};
     if ((rc = launch(g.dec_o, 64, 256, args, st))) return rc;
   }
   {
@@ -2038,7 +2041,7 @@ int qwen3_set_step_mode(int mode) {
   if (rc) return rc;
   if (mode == 1 && !g.step_capable)
     return fail(Q8_ERR_BAD_ARGUMENT, "this device cannot run the single-launch step "
-                "(needs its 448 workgroups resident at once, two per CU)");
+                "(needs its 512 workgroups resident at once, two per CU)");
   std::lock_guard<std::mutex> lock(g.mu);
   g.step_single = mode;
   return Q8_OK;
