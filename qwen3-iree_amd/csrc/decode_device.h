@@ -20,7 +20,12 @@ constexpr int kVocab = 151936;
 // kAttnShortCtx, where a split is at most two chunks of 32 positions; 64 above, where
 // the attention is bound by the bytes the waves have in flight (32 splits: 256
 // waves x 16 KiB, 1.63 us per chunk and wave, 2.6 TB/s).  Single-launch step
-// with 32 / 64 splits, context 2048 / 4096 / 8192 / 16384: LONG_FIGURES.
+// with 32 -> 64 splits, context 2049 / 4096 / 8192 / 16384: 618 -> 607, 673 ->
+// 632, 855 -> 745, 1219 -> 999 us; one layer's launches at 16384 40.2 -> 33.8.
+// At 1025 / 1536 / 2048 64 splits measured 568 / 570 / 573 against 559 / 571 /
+// 586 a step but 25.2-25.6 against 24.1-24.3 a layer (twice the partials to
+// merge).  Two chunks ahead with K rows straight to registers, without more
+// waves, was slower (1331 at 16384: the gathered row loads).
 constexpr int kAttnSplits = 32;
 constexpr int kAttnShortCtx = 2048;
 constexpr int kAttnWaves = 4;        // splits per workgroup, merged in LDS

@@ -648,7 +648,7 @@ constexpr int kVecWords = kAttnGroupsMax * 130;  // 2080: the largest polled vec
 // With split groups 8 .. 15 in the code (context 1024 / 16384): A 28 / 30 / 32
 // / 34 519 / 513 / 516 / 522 and 1016 / 1011 / 1008 / 1006, so A sleeps 30 where
 // a split is one chunk and 32 where the attention takes longer (2048: 592 at 30,
-// PACE2048 at 32); C 28 / 32 517-519, D 28 / 32 521 / 530, E 12 / 20 and the
+// 588 at 32); C 28 / 32 517-519, D 28 / 32 521 / 530, E 12 / 20 and the
 // cache chunk 4 / 12 within 1.
 #ifndef DEC_PACE_A
 #define DEC_PACE_A 30
