@@ -1065,6 +1065,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_attention(
 
   // several splits: (m, l, O) of this split's positions to its slot, row
   // 16 wave + c16; pf_attn_merge combines the slots
+  if (!qok) return;  // the merge reads the rows that exist
   float* slot = part + ((size_t)pair * kKvHeads + g) * kPfAttnSlotFloats;
   const int r = 16 * wave + c16;
 #pragma unroll

@@ -1576,22 +1576,36 @@ size_t pf_region_bytes(int32_t n, int i) {
 }
 
 // Positions per attention split, in blocks of 32.  A query block's positions
-// are walked one block after another, so without splits the longest query
-// block sets the time; each split costs a partial written and merged.  The
-// default is a third of the longest query block, at least 8 blocks: 8 (256
-// positions) measured best for 512-token prompts from position 0 (sweep of
-// 1 .. 24 and unsplit), 11 for 1024 tokens (3.218 ms against 3.249-3.317 for
-// 8-43) and 22 for 2048 (4.853 ms against 4.881-5.017 for 8-43).  Raised
-// where the partial slots would not hold the splits (4096 tokens: 32).
-constexpr int32_t kPfAttnSplitDefault = 8;
+// are walked one block after another (about 0.6 us each), so without splits
+// the longest query block sets the time; each split costs a partial written
+// and merged, and the first one the merge's launch.  nb = blocks of the longest
+// query block.
+//   No splits up to nb = 8, or 16 from 8 query blocks on (256 workgroups with
+//   the 8 kv heads): 300 tokens from position 0 (nb 10) 67.9 us a layer
+//   against 69.8 with splits of 8, 512 tokens (16) 69.9 against 70.2.
+//   From 32 query blocks on (1000 tokens) a third of nb, at least 8: flat
+//   within 2 % over 2 .. 32 blocks (1021 tokens 105.3 at 8, 2048 tokens 176.3
+//   at 22).
+//   Between, about 0.6 sqrt(nb), which balances the walk against the merge, at
+//   least 2, or 8 from 8 query blocks on.  Layer, against a third of nb: 1
+//   token after 300 / 1000 / 6000 positions 33.6 / 35.6 / 73.0 -> 29.4 / 32.2
+//   / 39.8 us, 33 tokens 40.2 / 47.2 (1700) / 79.0 -> 36.5 / 40.4 / 47.9, 100
+//   tokens after 6000 85.2 -> 60.0, 300 after 6000 114.6 -> 101.5.
+// Raised where the partial slots would not hold the splits.
+int32_t pf_attn_split_default(int32_t nqb, int32_t nb) {
+  if (nb <= (nqb >= 8 ? 16 : 8)) return nb;
+  if (nqb >= 32) return std::max(8, (nb + 2) / 3);
+  int32_t s = nqb >= 8 ? 8 : 2;
+  while (25LL * s * s < 9LL * nb) ++s;
+  return s;
+}
 
 int32_t pf_attn_split_blocks(int32_t n, int32_t p0, int chunk_local) {
   const PfSplitGeometry G = pf_split_geometry(n, p0, chunk_local ? p0 : 0);
   const int64_t cap = pf_attn_pair_cap(n);
   const int32_t nb_max = std::max(G.nb_last, G.c + G.nqb - 2);
   const int32_t set_split = g.pf_attn_split.load(std::memory_order_relaxed);
-  const int32_t s0 =
-      set_split > 0 ? set_split : std::max(kPfAttnSplitDefault, (nb_max + 2) / 3);
+  const int32_t s0 = set_split > 0 ? set_split : pf_attn_split_default(G.nqb, nb_max);
   int32_t lo_s = std::min(s0, nb_max), hi_s = nb_max;
   // smallest S >= lo_s whose pairs fit (at S = nb_max there are nqb pairs)
   while (lo_s < hi_s) {
