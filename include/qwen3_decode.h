@@ -231,8 +231,8 @@ int64_t qwen3_prefill_workspace_offset(int32_t n_tokens, const char* name);
 /* Work division of qwen3_prefill_batched / qwen3_prefill_layer (0 = the
  * default, for either):
  * gemm_rows: token rows per GEMM workgroup, 32, 64 or 128, where the tiled
- *   GEMMs run: attn_o, gate/up and ffn_down above 128 tokens, q/k/v above 256
- *   (below, row products whose tiles depend on the token count alone).  Over the Q8_0
+ *   GEMMs run, above 128 tokens (up to there, row products whose tiles depend
+ *   on the token count alone).  Over the Q8_0
  *   stacks: the q/k/v, attn_o and ffn_down GEMMs (gate/up always uses 64),
  *   32 or 64 (128 = 64); default: 32 where 64 would give fewer than 2
  *   workgroups per CU.  Over the f16 matrices: every GEMM, the tile of that

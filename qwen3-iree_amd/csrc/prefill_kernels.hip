@@ -3,27 +3,25 @@
 // :1731-2030) runs all prompt tokens of a layer together, so the layer
 // matrices become GEMMs [n_tokens, K] x [K, N] instead of n_tokens GEMVs.
 //
-// Per layer (eight launches, nine when an attention query block has several
-// position splits):
-//   pf_rmsnorm       rms_norm(h, attn_norm) of every token row
-//   pf_gemm_q8       q, k and v projections in one launch (MFMA, Q8_0 weights
-//                    dequantized to f16 in registers)
-//   pf_qk_rope_cache per-head rms_norm of q and k, RoPE at each token's
-//                    position, k and v written to their cache slots
+// Per layer:
+//   pf_rmsnorm       rms_norm(h, attn_norm) of every token row, and before the
+//                    first layer the RoPE table of the prompt's positions
+//   pf_gemm_*_qkv    q, k and v in one launch (MFMA; f16 weights, or Q8_0 ones
+//                    made f16 in registers), a head per tile: per-head
+//                    rms_norm, RoPE at each token's position and the k and v
+//                    cache slots written in the epilogue
 //   pf_attention     causal GQA attention of every token over the cache
-//   pf_attn_merge    the position splits' partial results combined
-//   pf_gemm_q8       attn_o + residual
-//   pf_rmsnorm       rms_norm(res, ffn_norm)
-//   pf_gemm_q8       gate/up with SwiGLU in the epilogue
-//   pf_gemm_q8       ffn_down + residual
+//   pf_attn_merge    the position splits' partial results combined (where a
+//                    query block has several)
+//   pf_gemm_*        attn_o (K in ranges), pf_res_reduce_norm their sum + residual
+//                    and rms_norm(res, ffn_norm)
+//   pf_gemm_*_swiglu gate/up with SwiGLU in the epilogue
+//   pf_gemm_*        ffn_down, pf_res_reduce[_norm] + residual (and the next
+//                    layer's rms_norm, inside a prompt)
 // plus pf_embed (token rows) before the first layer.  The vocab GEMV + argmax
 // of the last token reuses the decode kernels.  Up to 128 tokens the products
 // and norms are five launches of prefill_rows.h (four from 65 tokens on, with
-// RoPE in the q/k/v one, which runs up to 256).  Prompts of 129 to 1023 tokens
-// run attn_o and ffn_down with K split (pf_gemm_q8_part); their reduce
-// (pf_res_reduce_norm) then also forms the rms_norm that follows (ffn_norm of
-// the row after attn_o, the next layer's attn_norm after ffn_down), so those
-// two pf_rmsnorm launches drop out.
+// RoPE in the q/k/v one).
 //
 // Numerics follow the decode step op for op (f16 tensors between ops, f32 in
 // sums, norms and transcendental math): the norms, RoPE, SwiGLU and residual
@@ -34,10 +32,142 @@
 // weight is formed that way in registers (one f16 multiply of the exact
 // integer q by the f16 scale) and the MFMA accumulates f16 x * f16 w in f32,
 // over the whole K or over K ranges whose sums are added in order in f32.
+#include <type_traits>
+
 #include "decode_device.h"
 #include "prefill_split.h"
 
 namespace {
+
+// sq_tree4 and norm_pair with the conversions inside the arithmetic
+// (v_fma_mix_f32 widens an f16 operand exactly): the same bits, 20 instead of
+// 34 VALU instructions per 8 columns.  Squares of f16 values are exact in f32,
+// so fma(b, b, a a) is the sum of the two rounded squares; a product takes the
+// addend -0, which leaves every value and sign of zero as it is.
+__device__ __forceinline__ float sq_tree4_mix(uint32_t lo, uint32_t hi) {
+  float s[2];
+  const uint32_t v[2] = {lo, hi};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float a;
+    asm("v_fma_mix_f32 %0, %1, %1, neg(0) op_sel_hi:[1,1,0]" : "=v"(a) : "v"(v[i]));
+    asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]"
+        : "=v"(s[i])
+        : "v"(v[i]), "v"(a));
+  }
+  return s[0] + s[1];
+}
+__device__ __forceinline__ uint32_t norm_pair_mix(uint32_t h2, uint32_t w2, float inv) {
+  float a, b, x, y;
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[1,0,0]" : "=v"(a) : "v"(h2), "v"(inv));
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "=v"(b)
+      : "v"(h2), "v"(inv));
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[0,1,0]" : "=v"(x) : "v"(a), "v"(w2));
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,1,0] op_sel_hi:[0,1,0]"
+      : "=v"(y)
+      : "v"(b), "v"(w2));
+  return pack_f16x2(x, y);
+}
+
+// ------------------------------------------- head norms, RoPE, caches ----
+//
+// What follows the q/k/v product for one head of a tile of tokens: the head's
+// 128 columns are in LDS (f16, row r's 16-byte chunk c in slot c ^ (r & 15) of
+// its 256 bytes); per row the per-head rms_norm (q_norm / k_norm,
+// qwen3_full.mlir:1812-1879), RoPE at position start + token (:1060-1130) from
+// the table, and the cache writes (:1979-1983).  Sixteen lanes a row, lane j
+// holding dims 4 j .. + 3 and the dims 64 above, so a RoPE pair is in one lane
+// and the row's square root and reciprocal serve 8 dims a lane: about 110 VALU
+// instructions per 4 rows (one row per wave: 80 per row).  As its own launch
+// this read q, k and v back and took 4.8 / 6.2 / 10.6 us at 512 / 1021 / 2048
+// tokens, with 4-5 us for the table's.
+struct QkvOut {
+  uint16_t *q, *k, *v, *q_roped;
+  uint16_t *k_cache, *v_cache;  // the layer's base ([max_seq, 8, 128])
+  const uint16_t *qn_w, *kn_w;
+  const float* rope;  // [M][64 cosines, 64 sines]
+  int start;
+};
+
+// head: 0..15 q heads, 16..23 k, 24..31 v; rows m0 .. m0 + BM - 1 of M
+template <int BM, int THREADS>
+__device__ __forceinline__ void qkv_rope_rows(const QkvOut& A, const uint8_t* tile, int head,
+                                              int m0, int M) {
+  const int t = threadIdx.x;
+  const int j = t & 15;
+  const int kind = head < 16 ? 0 : (head < 24 ? 1 : 2);
+  const int hd = kind == 0 ? head : (head - 16) & 7;
+  uint2 w0 = {0, 0}, w1 = {0, 0};  // norm weights of dims 4 j .. and 64 + 4 j ..
+  if (kind != 2) {
+    const uint2* w = reinterpret_cast<const uint2*>(kind == 0 ? A.qn_w : A.kn_w) + j;
+    w0 = load_global(w);
+    w1 = load_global(w + 16);
+  }
+  uint16_t* raw = kind == 0 ? A.q : (kind == 1 ? A.k : A.v);
+  const int ld = kind == 0 ? 2048 : 1024;
+#pragma unroll 2
+  for (int r = t >> 4; r < BM; r += THREADS / 16) {
+    const int m = m0 + r;
+    if (m >= M) break;  // uniform over the row's 16 lanes; later rows are further out
+    const uint8_t* tr = tile + 256 * r + 8 * (j & 1);
+    const uint2 x0 = *reinterpret_cast<const uint2*>(tr + 16 * ((j >> 1) ^ (r & 15)));
+    const uint2 x1 = *reinterpret_cast<const uint2*>(tr + 16 * ((8 + (j >> 1)) ^ (r & 15)));
+    uint2* y = reinterpret_cast<uint2*>(raw + (size_t)m * ld + hd * kHeadDim) + j;
+    y[0] = x0;
+    y[16] = x1;
+    const size_t slot = ((size_t)(A.start + m) * kKvHeads + hd) * kHeadDim;
+    if (kind == 2) {
+      uint2* c = reinterpret_cast<uint2*>(A.v_cache + slot) + j;
+      c[0] = x0;
+      c[16] = x1;
+      continue;
+    }
+    const u32x4 cs4 = load_global(reinterpret_cast<const u32x4*>(A.rope + (size_t)m * 128) + j);
+    const u32x4 sn4 = load_global(reinterpret_cast<const u32x4*>(A.rope + (size_t)m * 128) + 16 + j);
+    const float ss = reduce_row16(sq_tree4_mix(x0.x, x0.y) + sq_tree4_mix(x1.x, x1.y));
+    const float inv = 1.0f / sqrtf(ss / 128.0f + kEps);
+    const uint32_t n0[2] = {norm_pair_mix(x0.x, w0.x, inv), norm_pair_mix(x0.y, w0.y, inv)};
+    const uint32_t n1[2] = {norm_pair_mix(x1.x, w1.x, inv), norm_pair_mix(x1.y, w1.y, inv)};
+    uint32_t o0[2], o1[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f16x2 a2 = as_f16x2(n0[h]), b2 = as_f16x2(n1[h]);
+      float lo[2], hi[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float a = (float)a2[e], b = (float)b2[e];
+        // copy out first: a bit cast of a vector element lvalue reads element 0
+        const uint32_t cb = cs4[2 * h + e], sb = sn4[2 * h + e];
+        const float c = __uint_as_float(cb), s = __uint_as_float(sb);
+        const float ac = a * c, bs = b * s, as = a * s, bc = b * c;
+        lo[e] = ac - bs;
+        hi[e] = as + bc;
+      }
+      o0[h] = pack_f16x2(lo[0], lo[1]);
+      o1[h] = pack_f16x2(hi[0], hi[1]);
+    }
+    uint2* z = reinterpret_cast<uint2*>(kind == 0 ? A.q_roped + (size_t)m * 2048 + hd * kHeadDim
+                                                  : A.k_cache + slot) +
+               j;
+    z[0] = (uint2){o0[0], o0[1]};
+    z[16] = (uint2){o1[0], o1[1]};
+  }
+}
+
+// One 16 x 16 accumulator tile (rows r0 .., columns c0 .. of the head) into
+// that LDS tile.
+__device__ __forceinline__ void qkv_tile_store(uint8_t* tile, int r0, int c0, f32x4 acc) {
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, col = c0 + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + 4 * g + i;
+    const float v = acc[i];
+    *reinterpret_cast<uint16_t*>(tile + 256 * r + 16 * ((col >> 3) ^ (r & 15)) + 2 * (col & 7)) =
+        f32_to_f16_bits(v);
+  }
+}
 
 // ---------------------------------------------------------------- GEMM ----
 //
@@ -54,14 +184,11 @@ namespace {
 // (k / 8), element k % 8; B[k][j] in lane j + 16 (k / 8), element k % 8;
 // C[i][j] in lane j + 16 (i / 4), element i % 4.
 
-constexpr int kGemmBN = 64;
 constexpr int kStageBlocks = 8;
 constexpr int kXRow = 2 * 32 * kStageBlocks + 16;  // 528
 constexpr int kWRow = 34 * kStageBlocks;           // 272
-constexpr int kWLds = kGemmBN * kWRow;
-constexpr int kWPieces = kGemmBN * 17;
 
-enum { kEpiStore = 0, kEpiResidual = 1, kEpiSwiGLU = 2, kEpiPartial = 3 };
+enum { kEpiQkv = 0, kEpiResidual = 1, kEpiSwiGLU = 2, kEpiPartial = 3 };
 
 struct GemmArgs {
   const uint16_t* x;  // [M, ldx] f16
@@ -72,14 +199,9 @@ struct GemmArgs {
   int n_tiles;        // output tiles of 64 columns (kEpiSwiGLU: 32 gate + 32 up rows)
   int ldx, ldy, ldr;
   int up_row;         // kEpiSwiGLU: first up row of W (gate rows are 0..up_row-1)
-  // Up to three products with the same x in one launch: tiles [seg_tile[0],
-  // seg_tile[1]) use w_seg[0] / y_seg[0] / ldy_seg[0], tiles from seg_tile[1]
-  // on the second set (tile numbers counted from the set's first tile);
-  // seg_tile = n_tiles when unused.
-  const uint8_t* w_seg[2];
-  uint16_t* y_seg[2];
-  int ldy_seg[2];
-  int seg_tile[2];
+  // kEpiQkv: w the q rows, then these (a tile is a head: 16 q, 8 k, 8 v)
+  const uint8_t *wk, *wv;
+  QkvOut qkv;
   // kEpiPartial: K in `splits` equal ranges, one per group of workgroups;
   // split s stores its f32 sums at part[(s M + m) N + n], N = 64 n_tiles
   float* part;
@@ -89,6 +211,9 @@ struct GemmArgs {
 template <int EPI, int BM>
 __device__ __forceinline__ void gemm_q8(const GemmArgs& A) {
   static_assert(BM == 64 || (BM == 32 && EPI != kEpiSwiGLU), "tile shapes");
+  constexpr int kGemmBN = EPI == kEpiQkv ? 128 : 64;
+  constexpr int kWLds = kGemmBN * kWRow;
+  constexpr int kWPieces = kGemmBN * 17;
   constexpr int kXL = BM * kXRow;
   constexpr int kXP = BM * 32;   // 16-byte X pieces per stage
   // waves 2 (m) x 2 (n) of 32 x 32 (SwiGLU: 32 tokens x 16 gate + 16 up
@@ -96,7 +221,7 @@ __device__ __forceinline__ void gemm_q8(const GemmArgs& A) {
   // once and uses it for all BM / 16 of its m tiles
   constexpr bool kSplitM = EPI == kEpiSwiGLU;
   constexpr int MS = kSplitM ? 2 : BM / 16;  // 16-row tiles per wave
-  constexpr int NS = kSplitM ? 2 : 1;        // 16-column tiles per wave
+  constexpr int NS = kSplitM || EPI == kEpiQkv ? 2 : 1;  // 16-column tiles per wave
   __shared__ __attribute__((aligned(16))) uint8_t lds[kXL + kWLds];
   uint8_t* xl = lds;
   uint8_t* wl = lds + kXL;
@@ -119,13 +244,13 @@ __device__ __forceinline__ void gemm_q8(const GemmArgs& A) {
   const int m0 = (slot % mt) * BM;
   const uint8_t* wb = A.w;
   uint16_t* yb = A.y;
-  int ldy = A.ldy;
-  if (n_tile >= A.seg_tile[0]) {
-    const int sg = n_tile >= A.seg_tile[1] ? 1 : 0;
-    wb = A.w_seg[sg];
-    yb = A.y_seg[sg];
-    ldy = A.ldy_seg[sg];
-    n_tile -= A.seg_tile[sg];
+  const int ldy = A.ldy;
+  const int head = n_tile;
+  if constexpr (EPI == kEpiQkv) {
+    if (n_tile >= 16) {
+      wb = n_tile < 24 ? A.wk : A.wv;
+      n_tile = (n_tile - 16) & 7;
+    }
   }
   const int row_bytes = A.K / 32 * 34;
   const int stages = A.K / (32 * kStageBlocks) / (EPI == kEpiPartial ? A.splits : 1);
@@ -181,7 +306,8 @@ __device__ __forceinline__ void gemm_q8(const GemmArgs& A) {
     nrow[0] = 16 * wn + c16;       // gate row
     nrow[1] = 32 + 16 * wn + c16;  // the matching up row
   } else {
-    nrow[0] = 16 * wn + c16;
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns) nrow[ns] = 16 * NS * wn + 16 * ns + c16;
   }
   f32x4 acc[MS][NS];
 #pragma unroll
@@ -235,6 +361,17 @@ __device__ __forceinline__ void gemm_q8(const GemmArgs& A) {
     }
   }
 
+  if constexpr (EPI == kEpiQkv) {
+    __syncthreads();  // every wave is done reading the last stage
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns)
+        qkv_tile_store(lds, 16 * ms, 16 * NS * wn + 16 * ns, acc[ms][ns]);
+    __syncthreads();
+    qkv_rope_rows<BM, 256>(A.qkv, lds, head, m0, A.M);
+    return;
+  }
   // epilogue: lane holds rows 4 g + i, column c16 of each 16 x 16 tile
 #pragma unroll
   for (int ms = 0; ms < MS; ++ms) {
@@ -302,12 +439,7 @@ struct GemmF16Args {
   int n_tiles;        // tiles of BN columns of W
   int ldx, ldy, ldr;
   int splits;         // kEpiPartial: K in `splits` equal ranges
-  // output columns [seg_col[0], seg_col[1]) go to y_seg[0] (ld ldy_seg[0]),
-  // columns from seg_col[1] on to y_seg[1], each counted from its first;
-  // seg_col = N when unused
-  uint16_t* y_seg[2];
-  int ldy_seg[2];
-  int seg_col[2];
+  QkvOut qkv;         // kEpiQkv: a tile is a head's 128 columns
 };
 
 // byte offset of row r's 16-byte chunk c (k 8 c .. 8 c + 7 of the stage) in
@@ -320,6 +452,61 @@ __device__ __forceinline__ int f16_lds_off(int r, int c) {
     static_assert(C == 8, "row length");
     const int line = r >> 1;
     return 256 * line + 16 * ((((r & 1) << 3) | c) ^ (line & 15));
+  }
+}
+
+// The tile's results out of the accumulators (wave (wm, wn) of WM x WN holds 16
+// MS x 16 NS of them, lane rows 4 g + i, column c16 of each 16 x 16 piece).
+// tile: LDS of 256 bytes per token row for kEpiQkv.
+template <int EPI, int MS, int NS, int WM, int WN, int kTileBytes>
+__device__ __forceinline__ void gemm_f16_epilogue(const GemmF16Args& A, const f32x4 (&acc)[MS][NS],
+                                                  uint8_t* tile, int m0, int n_tile, int split) {
+  constexpr int BM = 16 * MS * WM, BN = 16 * NS * WN;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, c16 = lane & 15;
+  const int wm = wave % WM, wn = wave / WM;
+  if constexpr (EPI == kEpiQkv) {
+    static_assert(BN == 128, "a head per tile");
+    static_assert(256 * BM <= kTileBytes, "the head's rows in the first stage buffer");
+    __syncthreads();  // every wave is done reading the last stage
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns)
+        qkv_tile_store(tile, 16 * MS * wm + 16 * ms, 16 * NS * wn + 16 * ns, acc[ms][ns]);
+    __syncthreads();
+    qkv_rope_rows<BM, 64 * WM * WN>(A.qkv, tile, n_tile, m0, A.M);
+    return;
+  }
+  const int N = BN * A.n_tiles;
+  const int col0 = BN * n_tile + 16 * NS * wn;
+#pragma unroll
+  for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + 16 * MS * wm + 16 * ms + 4 * g + i;
+      if (m >= A.M) continue;
+      if constexpr (EPI == kEpiSwiGLU) {
+        // W rows come in groups of 32: 16 gate rows, then the matching 16 up
+        // rows (pf_expand_q8's gate/up order); group G feeds columns 16 G ..
+#pragma unroll
+        for (int p = 0; p < NS / 2; ++p) {
+          const int col = (col0 + 32 * p) / 2 + c16;
+          A.y[(size_t)m * A.ldy + col] = swiglu_f16(acc[ms][2 * p][i], acc[ms][2 * p + 1][i]);
+        }
+      } else {
+#pragma unroll
+        for (int ns = 0; ns < NS; ++ns) {
+          const int col = col0 + 16 * ns + c16;
+          if constexpr (EPI == kEpiResidual)
+            A.y[(size_t)m * A.ldy + col] =
+                residual_f16(as_half(A.r[(size_t)m * A.ldr + col]), acc[ms][ns][i]);
+          else
+            A.part[((size_t)split * A.M + m) * N + col] = acc[ms][ns][i];
+        }
+      }
+    }
   }
 }
 
@@ -467,48 +654,159 @@ __device__ __forceinline__ void gemm_f16(const GemmF16Args& A) {
     }
   }
 
-  // epilogue: lane holds rows 4 g + i, column c16 of each 16 x 16 piece
-  const int N = BN * A.n_tiles;
-  int col0 = n0 + 16 * NS * wn;
-  uint16_t* yb = A.y;
-  int ldy = A.ldy;
-  if constexpr (EPI == kEpiStore) {
-    if (n0 >= A.seg_col[0]) {
-      const int sg = n0 >= A.seg_col[1] ? 1 : 0;
-      yb = A.y_seg[sg];
-      ldy = A.ldy_seg[sg];
-      col0 -= A.seg_col[sg];
+  gemm_f16_epilogue<EPI, MS, NS, WM, WN, kBuf>(A, acc, lds0, m0, n_tile, split);
+}
+
+// The same product with NBUF stages of 64 k in LDS and the fragments of the next
+// 32 k read while the current ones are multiplied, for a workgroup alone on its
+// CU: where the grid gives a CU no second workgroup to hide behind, copies
+// have to run several stages ahead, past bare s_barriers (__syncthreads would
+// drain them).  q/k/v at 512 tokens (256 workgroups of 64 x 128): 8.0-8.8 us
+// with six stages and eight waves against 9.7-11.0 for 64 x 64 tiles, two per
+// CU, with two.  With two workgroups a CU the two-buffer form above stays
+// faster (2048 tokens, 128 x 128: 22 us against 25).  The compiler counts
+// global_load_lds against lgkmcnt too, so each half waits for its LDS reads
+// (issued 16 MFMAs earlier) before the copies go out.
+template <int N, class F, int I = 0>
+__device__ __forceinline__ void pf_static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    pf_static_for<N, F, I + 1>(static_cast<F&&>(f));
+  }
+}
+
+template <int EPI, int STAGES, int MS, int NS, int NBUF, int WM, int WN>
+__device__ __forceinline__ void gemm_pipe(const GemmF16Args& A) {
+  static_assert(NBUF >= 3 && NBUF <= 6, "buffers");
+  constexpr int KS = 64;
+  constexpr int kWaves = WM * WN;
+  constexpr int BM = 16 * MS * WM, BN = 16 * NS * WN;
+  constexpr int kRows = BM + BN;
+  constexpr int RB = 2 * KS;
+  constexpr int C = RB / 16;
+  constexpr int J = kRows / 8 / kWaves;  // copy instructions per wave per stage
+  static_assert(kRows % (8 * kWaves) == 0, "copy pieces");
+  constexpr int kBuf = kRows * RB;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds0[kBuf];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds1[kBuf];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds2[kBuf];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds3[NBUF > 3 ? kBuf : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds4[NBUF > 4 ? kBuf : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds5[NBUF > 5 ? kBuf : 16];
+  uint8_t* const bufs[6] = {lds0, lds1, lds2, lds3, lds4, lds5};
+  const int t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lane = t & 63;
+  const int g = lane >> 4;
+  const int c16 = lane & 15;
+  const int mt = (A.M + BM - 1) / BM;
+  const int tiles = mt * A.n_tiles;
+  const int split = EPI == kEpiPartial ? (int)blockIdx.x / tiles : 0;
+  const int bid = (int)blockIdx.x - split * tiles;
+  const int xcd = bid & 7;
+  const int slot = bid >> 3;
+  const int n_tile = (slot / mt) * 8 + xcd;
+  const int m0 = (slot % mt) * BM;
+  const int n0 = n_tile * BN;
+  const int k0 = split * STAGES * KS;
+  const uint8_t* src[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int line = 4 * (J * wave + j) + (lane >> 4);
+    const int p = (lane & 15) ^ (line & 15);
+    const int row = 2 * line + (p >> 3);
+    const int kc = p & 7;
+    if (row < BM) {
+      const int m = m0 + row < A.M ? m0 + row : A.M - 1;
+      src[j] = reinterpret_cast<const uint8_t*>(A.x + (size_t)m * A.ldx + k0) + 16 * kc;
+    } else {
+      src[j] = reinterpret_cast<const uint8_t*>(A.w + (size_t)(n0 + row - BM) * A.K + k0) + 16 * kc;
     }
   }
+  auto issue = [&](int s, uint8_t* buf) {
 #pragma unroll
-  for (int ms = 0; ms < MS; ++ms) {
+    for (int j = 0; j < J; ++j)
+      __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)(src[j] + RB * s),
+                                       (LDS_AS void*)(buf + 1024 * (J * wave + j)), 16, 0, 0);
+  };
+  const int wm = wave % WM;
+  const int wn = wave / WM;
+  int off[2][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + 16 * MS * wm + 16 * ms + 4 * g + i;
-      if (m >= A.M) continue;
-      if constexpr (EPI == kEpiSwiGLU) {
-        // W rows come in groups of 32: 16 gate rows, then the matching 16 up
-        // rows (pf_expand_q8's gate/up order); group G feeds columns 16 G ..
+  for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-        for (int p = 0; p < NS / 2; ++p) {
-          const int col = (col0 + 32 * p) / 2 + c16;
-          yb[(size_t)m * ldy + col] = swiglu_f16(acc[ms][2 * p][i], acc[ms][2 * p + 1][i]);
-        }
-      } else {
+    for (int kb = 0; kb < 2; ++kb)
+      off[hb][kb] = f16_lds_off<C>(16 * hb + c16, 4 * kb + g) - 16 * C * 16 * hb;
+  static_assert(MS % 2 == 0 && NS % 2 == 0, "fragment row bases");
+  f32x4 acc[MS][NS];
 #pragma unroll
-        for (int ns = 0; ns < NS; ++ns) {
-          const int col = col0 + 16 * ns + c16;
-          if constexpr (EPI == kEpiResidual)
-            yb[(size_t)m * ldy + col] =
-                residual_f16(as_half(A.r[(size_t)m * A.ldr + col]), acc[ms][ns][i]);
-          else if constexpr (EPI == kEpiPartial)
-            A.part[((size_t)split * A.M + m) * N + col] = acc[ms][ns][i];
-          else
-            yb[(size_t)m * ldy + col] = f32_to_f16_bits(acc[ms][ns][i]);
-        }
-      }
+  for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  f16x8 a[2][MS], b[2][NS];
+  auto read = [&](const uint8_t* buf, int kb) {
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+      a[kb][ms] = *reinterpret_cast<const f16x8*>(buf + (16 * MS * wm + 16 * ms) * RB + off[ms & 1][kb]);
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns)
+      b[kb][ns] = *reinterpret_cast<const f16x8*>(buf + (BM + 16 * NS * wn + 16 * ns) * RB + off[ns & 1][kb]);
+  };
+  auto mul = [&](int kb) {
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns)
+        acc[ms][ns] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[kb][ms], b[kb][ns], acc[ms][ns], 0, 0, 0);
+  };
+  auto bar = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  static_assert(STAGES >= 2 * NBUF, "stages");
+#pragma unroll
+  for (int i = 0; i < NBUF - 1; ++i) issue(i, bufs[i]);
+  wait_vm<J * (NBUF - 2)>();
+  bar();
+  read(lds0, 0);
+  // stage s out of cur; LEFT >= 0: stages after it (the tail), -1: at least
+  // NBUF - 1
+  auto step = [&](auto left, int s, const uint8_t* cur, const uint8_t* next, uint8_t* refill) {
+    constexpr int kLeft = decltype(left)::value;
+    wait_lds();
+    read(cur, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_lds();
+    if constexpr (kLeft != 0) {
+      // stage s + 1 has landed: only the stages behind it may be out
+      constexpr int kOut = kLeft < 0 || kLeft > NBUF - 2 ? NBUF - 3 : kLeft - 1;
+      wait_vm<J * kOut>();
+      bar();
+      if constexpr (kLeft < 0) issue(s + NBUF - 1, refill);
+      read(next, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    mul(1);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int kMain = (STAGES - (NBUF - 1)) / NBUF * NBUF;  // stages of the loop
+  for (int s = 0; s < kMain; s += NBUF) {
+#pragma unroll
+    for (int i = 0; i < NBUF; ++i)
+      step(std::integral_constant<int, -1>{}, s + i, bufs[i], bufs[(i + 1) % NBUF],
+           bufs[(i + NBUF - 1) % NBUF]);
   }
+  pf_static_for<STAGES - kMain>([&](auto i) {
+    constexpr int kI = decltype(i)::value;
+    constexpr int kLeft = STAGES - kMain - 1 - kI;
+    step(std::integral_constant<int, (kLeft >= NBUF - 1 ? -1 : kLeft)>{}, kMain + kI,
+         bufs[kI % NBUF], bufs[(kI + 1) % NBUF], bufs[(kI + NBUF - 1) % NBUF]);
+  });
+
+  gemm_f16_epilogue<EPI, MS, NS, WM, WN, kBuf>(A, acc, lds0, m0, n_tile, split);
 }
 
 }  // namespace
@@ -571,27 +869,60 @@ extern "C" __global__ __launch_bounds__(128) void pf_embed(const int32_t* __rest
 }
 
 // out[i] = rms_norm(h[i], w) (qwen3_full.mlir:96-133, the same computation as
-// @rms_norm_1x1024): 16 lanes per row, the decode step's lane layout and
-// reduction, so a row's result is the decode kernels' bit for bit.
-extern "C" __global__ __launch_bounds__(256) void pf_rmsnorm(const uint16_t* __restrict__ h,
-                                                             const uint16_t* __restrict__ w,
-                                                             uint16_t* __restrict__ out, int n) {
-  const int row = blockIdx.x * 16 + (threadIdx.x >> 4);
+// @rms_norm_1x1024): 4 rows a workgroup of one wave, 16 lanes a row, lane p
+// holding chunks p + 16 i of 8 columns (contiguous loads), the squares summed
+// in the canonical order, so a row's result is the decode kernels' bit for
+// bit.  Workgroups from (n + 3) / 4 on write the RoPE table of the prompt's
+// positions instead, four tokens each: table[i] = the 64 cosines then the 64
+// sines of the angles at position start + i (rope_angle: the decode step's
+// values), for every layer of a prompt.
+extern "C" __global__ __launch_bounds__(64) void pf_rmsnorm(const uint16_t* __restrict__ h,
+                                                            const uint16_t* __restrict__ w,
+                                                            uint16_t* __restrict__ out, int n,
+                                                            int start, float* __restrict__ table) {
+  const int lane = threadIdx.x;
+  const int norm_wgs = (n + 3) / 4;
+  if ((int)blockIdx.x >= norm_wgs) {
+    const int i0 = 4 * ((int)blockIdx.x - norm_wgs);
+    for (int i = i0; i < i0 + 4 && i < n; ++i) {
+      float c, s;
+      rope_angle(start + i, lane, c, s);
+      table[(size_t)i * 128 + lane] = c;
+      table[(size_t)i * 128 + 64 + lane] = s;
+    }
+    return;
+  }
+  const int row = 4 * blockIdx.x + (lane >> 4);
   const int r = row < n ? row : n - 1;
-  u32x4 xr[8];
-  rmsnorm_gemv_x<false>(h + (size_t)r * kHidden, w, xr);
-  if (row < n) {
-    u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)r * kHidden + 64 * (threadIdx.x & 15));
+  const int p = lane & 15;
+  u32x4 hv[8], wv[8];
 #pragma unroll
-    for (int m = 0; m < 8; ++m) o[m] = xr[m];
+  for (int i = 0; i < 8; ++i)
+    hv[i] = load_global(reinterpret_cast<const u32x4*>(h + (size_t)r * kHidden) + p + 16 * i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) wv[i] = load_global(reinterpret_cast<const u32x4*>(w) + p + 16 * i);
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    s[i] = reduce_row16(sq_tree4_mix(hv[i][0], hv[i][1]) + sq_tree4_mix(hv[i][2], hv[i][3]));
+  const float inv = rms_inv(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])));
+  if (row < n) {
+    u32x4* o = reinterpret_cast<u32x4*>(out + (size_t)row * kHidden) + p;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      u32x4 x;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = norm_pair_mix(hv[i][j], wv[i][j], inv);
+      o[16 * i] = x;
+    }
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8(GemmArgs A) {
-  gemm_q8<kEpiStore, 64>(A);
+extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_qkv(GemmArgs A) {
+  gemm_q8<kEpiQkv, 64>(A);
 }
-extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_m32(GemmArgs A) {
-  gemm_q8<kEpiStore, 32>(A);
+extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_qkv_m32(GemmArgs A) {
+  gemm_q8<kEpiQkv, 32>(A);
 }
 extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_res(GemmArgs A) {
   gemm_q8<kEpiResidual, 64>(A);
@@ -667,7 +998,7 @@ extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_swiglu(GemmArgs A) 
 // tokens x 32 NS columns of W per workgroup (four waves); the stage length and buffer
 // count are the fastest measured for where the host uses each (cold weights,
 // 512-2048 tokens): 64 k for the 128-column tiles (two workgroups per CU);
-// 128 k for the 64 x 64 tiles of q/k/v and attn_o / ffn_down with two
+// 128 k for the 64 x 64 tiles of attn_o / ffn_down with two
 // workgroups per CU, 256 k (the "k" names: 128 KiB of LDS, one workgroup per
 // CU) where the grid covers the CUs once; the SwiGLU 64 x 64 tile keeps 64 k.
 #define PF_GEMM_F16(name, EPI, MS, NS, KS, NBUF)                          \
@@ -680,9 +1011,11 @@ extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_swiglu(GemmArgs A) 
 extern "C" __global__ __launch_bounds__(512) void pf_gemm_f16_swiglu_46w(GemmF16Args A) {
   gemm_f16<kEpiSwiGLU, 4, 6, 64, 2, 4, 2>(A);
 }
-PF_GEMM_F16(pf_gemm_f16_44, kEpiStore, 4, 4, 64, 2)
-PF_GEMM_F16(pf_gemm_f16_24, kEpiStore, 2, 4, 64, 2)
-PF_GEMM_F16(pf_gemm_f16_22, kEpiStore, 2, 2, 128, 2)
+PF_GEMM_F16(pf_gemm_f16_qkv_44, kEpiQkv, 4, 4, 64, 2)
+PF_GEMM_F16(pf_gemm_f16_qkv_24, kEpiQkv, 2, 4, 64, 2)
+extern "C" __global__ __launch_bounds__(512) void pf_gemm_f16_qkv_22p(GemmF16Args A) {
+  gemm_pipe<kEpiQkv, 16, 2, 2, 6, 2, 4>(A);
+}
 PF_GEMM_F16(pf_gemm_f16_swiglu_44, kEpiSwiGLU, 4, 4, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_swiglu_24, kEpiSwiGLU, 2, 4, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_swiglu_22, kEpiSwiGLU, 2, 2, 64, 2)
@@ -743,17 +1076,6 @@ __device__ __forceinline__ void rope_lane(const float* __restrict__ rope, int m,
   cs[1] = __uint_as_float(c2.y);
   sn[0] = __uint_as_float(s2.x);
   sn[1] = __uint_as_float(s2.y);
-}
-
-// table[i] = the 64 cosines then the 64 sines of the RoPE angles at position
-// start + i (rope_angle: the decode step's values), for every layer of a
-// prompt.  One 64-lane workgroup per token.
-extern "C" __global__ __launch_bounds__(64) void pf_rope_table(int start, float* __restrict__ table) {
-  const int i = blockIdx.x, lane = threadIdx.x;
-  float c, s;
-  rope_angle(start + i, lane, c, s);
-  table[(size_t)i * 128 + lane] = c;
-  table[(size_t)i * 128 + 64 + lane] = s;
 }
 
 #include "prefill_rows.h"

@@ -1,4 +1,4 @@
-// Products of a short prompt's layer (up to 128 tokens, q/k/v up to 256), each
+// Products of a short prompt's layer (up to 128 tokens), each
 // workgroup holding the whole K of its few weight rows ("row products"),
 // included by prefill_kernels.hip.
 //
@@ -118,37 +118,6 @@ constexpr int kRowBytes1024 = Q8 ? 1088 : 2048;  // bytes of 1024 k of a weight 
 // rows: slot c ^ (r & 15) of each 256 bytes, so a fragment read (16 rows, one
 // chunk) touches 16 slots and so does a row write (16 lanes, 16 chunks).
 __device__ __forceinline__ int rows_off(int r, int c) { return 2048 * r + 16 * (c ^ (r & 15)); }
-
-// sq_tree4 and norm_pair with the conversions inside the arithmetic
-// (v_fma_mix_f32 widens an f16 operand exactly): the same bits, 20 instead of
-// 34 VALU instructions per 8 columns.  Squares of f16 values are exact in f32,
-// so fma(b, b, a a) is the sum of the two rounded squares; a product takes the
-// addend -0, which leaves every value and sign of zero as it is.
-__device__ __forceinline__ float sq_tree4_mix(uint32_t lo, uint32_t hi) {
-  float s[2];
-  const uint32_t v[2] = {lo, hi};
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    float a;
-    asm("v_fma_mix_f32 %0, %1, %1, neg(0) op_sel_hi:[1,1,0]" : "=v"(a) : "v"(v[i]));
-    asm("v_fma_mix_f32 %0, %1, %1, %2 op_sel:[1,1,0] op_sel_hi:[1,1,0]"
-        : "=v"(s[i])
-        : "v"(v[i]), "v"(a));
-  }
-  return s[0] + s[1];
-}
-__device__ __forceinline__ uint32_t norm_pair_mix(uint32_t h2, uint32_t w2, float inv) {
-  float a, b, x, y;
-  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[1,0,0]" : "=v"(a) : "v"(h2), "v"(inv));
-  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-      : "=v"(b)
-      : "v"(h2), "v"(inv));
-  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[0,1,0]" : "=v"(x) : "v"(a), "v"(w2));
-  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,1,0] op_sel_hi:[0,1,0]"
-      : "=v"(y)
-      : "v"(b), "v"(w2));
-  return pack_f16x2(x, y);
-}
 
 // xl rows 0 .. 16 MS - 1 = rms_norm(h[m0 + row], w) (rows past M repeat row
 // M - 1).  16 lanes per row, lane p holding chunks p + 16 i, so loads and LDS
@@ -608,11 +577,8 @@ __device__ __forceinline__ void rows_res(const RowsResArgs& A) {
 // how many tokens.
 #define PF_ROWS(name, threads, Args, ...) \
   extern "C" __global__ __launch_bounds__(threads) void name(Args A) { __VA_ARGS__(A); }
-#define PF_ROWS_QKV_ROPE(MS)                                                                 \
-  PF_ROWS(pf_rows_qkv_rope_##MS, 512, RowsQkvArgs, rows_qkv<false, MS>)                      \
-  PF_ROWS(pf_rows_qkv_rope_q8_##MS, 512, RowsQkvArgs, rows_qkv<true, MS>)
-PF_ROWS_QKV_ROPE(1)
-PF_ROWS_QKV_ROPE(2)
+PF_ROWS(pf_rows_qkv_rope, 512, RowsQkvArgs, rows_qkv<false, 1>)
+PF_ROWS(pf_rows_qkv_rope_q8, 512, RowsQkvArgs, rows_qkv<true, 1>)
 #define PF_ROWS_QKV(MS, NS)                                                                  \
   PF_ROWS(pf_rows_qkv_##MS##NS, 512, RowsNormArgs, rows_norm<false, false, MS, NS>)          \
   PF_ROWS(pf_rows_qkv_q8_##MS##NS, 512, RowsNormArgs, rows_norm<false, true, MS, NS>)
@@ -632,7 +598,6 @@ PF_ROWS_GU(2, 6)
   PF_ROWS(pf_rows_dn_q8_##MS, 768, RowsResArgs, rows_res<true, MS, 12>)
 PF_ROWS_RES(1)
 PF_ROWS_RES(2)
-#undef PF_ROWS_QKV_ROPE
 #undef PF_ROWS_QKV
 #undef PF_ROWS_GU
 #undef PF_ROWS_RES

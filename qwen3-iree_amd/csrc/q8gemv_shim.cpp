@@ -117,14 +117,15 @@ struct State {
                 dec_o = nullptr, dec_gu = nullptr, dec_dn = nullptr, dec_vocab = nullptr,
                 dec_final = nullptr, dec_adv = nullptr, dec_clear = nullptr, dec_step = nullptr;
   hipModule_t pf_module = nullptr;  // prefill_gfx950.hsaco (optional)
-  hipFunction_t pf_embed = nullptr, pf_norm = nullptr, pf_gemm = nullptr, pf_gemm_res = nullptr,
-                pf_gemm_m32 = nullptr, pf_gemm_res_m32 = nullptr, pf_gemm_swiglu = nullptr,
+  hipFunction_t pf_embed = nullptr, pf_norm = nullptr, pf_gemm_qkv = nullptr, pf_gemm_res = nullptr,
+                pf_gemm_qkv_m32 = nullptr, pf_gemm_res_m32 = nullptr, pf_gemm_swiglu = nullptr,
                 pf_gemm_part = nullptr, pf_gemm_part_m32 = nullptr, pf_res_reduce = nullptr,
-                pf_res_reduce_norm = nullptr, pf_rope = nullptr, pf_rope_table = nullptr,
+                pf_res_reduce_norm = nullptr, pf_rope = nullptr,
                 pf_attn = nullptr, pf_attn_merge = nullptr, pf_set_pos = nullptr;
   // the f16 GEMMs (pf_gemm_f16*: over the f16 layer matrices) and their
   // expansion from Q8_0 (pf_expand_q8)
-  hipFunction_t pf_f16_44 = nullptr, pf_f16_24 = nullptr, pf_f16_22 = nullptr,
+  hipFunction_t pf_f16_qkv_44 = nullptr, pf_f16_qkv_24 = nullptr,
+                pf_f16_qkv_22p = nullptr,
                 pf_f16_sw_46w = nullptr, pf_f16_sw_44 = nullptr, pf_f16_sw_24 = nullptr,
                 pf_f16_sw_22 = nullptr,
                 pf_f16_res_22 = nullptr, pf_f16_res_22k = nullptr, pf_f16_res_12k = nullptr,
@@ -132,7 +133,7 @@ struct State {
                 pf_f16_part_44 = nullptr, pf_f16_part_44k = nullptr, pf_expand = nullptr;
   // the row products (prefill_rows.h): [instance, fewest tokens first][0: f16
   // weights, 1: Q8_0]
-  hipFunction_t pf_rows_qkv_rope[2][2] = {}, pf_rows_qkv[2][2] = {}, pf_rows_gu[4][2] = {},
+  hipFunction_t pf_rows_qkv_rope[2] = {}, pf_rows_qkv[2][2] = {}, pf_rows_gu[4][2] = {},
                 pf_rows_o[2][2] = {}, pf_rows_dn[2][2] = {};
   std::atomic<int> pf_tile_rows{0};   // prefill GEMM token tile: 0 = by shape, 32, 64 or 128
   std::atomic<int> pf_attn_split{0};  // prefill attention positions per split in blocks of 32
@@ -364,12 +365,12 @@ int q8gemv_init(const char* code_object_path) {
           const char* name;
         } names[] = {{&g.pf_embed, "pf_embed"},
                      {&g.pf_norm, "pf_rmsnorm"},
-                     {&g.pf_gemm, "pf_gemm_q8"},
+                     {&g.pf_gemm_qkv, "pf_gemm_q8_qkv"},
                      {&g.pf_gemm_res, "pf_gemm_q8_res"},
-                     {&g.pf_gemm_m32, "pf_gemm_q8_m32"},
+                     {&g.pf_gemm_qkv_m32, "pf_gemm_q8_qkv_m32"},
                      {&g.pf_gemm_res_m32, "pf_gemm_q8_res_m32"},
                      {&g.pf_gemm_swiglu, "pf_gemm_q8_swiglu"},
-                     {&g.pf_rope, "pf_qk_rope_cache"}, {&g.pf_rope_table, "pf_rope_table"},
+                     {&g.pf_rope, "pf_qk_rope_cache"},
                      {&g.pf_attn, "pf_attention"},
                      {&g.pf_attn_merge, "pf_attn_merge"},
                      {&g.pf_gemm_part, "pf_gemm_q8_part"},
@@ -377,9 +378,9 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_res_reduce, "pf_res_reduce"},
                      {&g.pf_res_reduce_norm, "pf_res_reduce_norm"},
                      {&g.pf_set_pos, "pf_set_pos"},
-                     {&g.pf_f16_44, "pf_gemm_f16_44"},
-                     {&g.pf_f16_24, "pf_gemm_f16_24"},
-                     {&g.pf_f16_22, "pf_gemm_f16_22"},
+                     {&g.pf_f16_qkv_44, "pf_gemm_f16_qkv_44"},
+                     {&g.pf_f16_qkv_24, "pf_gemm_f16_qkv_24"},
+                     {&g.pf_f16_qkv_22p, "pf_gemm_f16_qkv_22p"},
                      {&g.pf_f16_sw_46w, "pf_gemm_f16_swiglu_46w"},
                      {&g.pf_f16_sw_44, "pf_gemm_f16_swiglu_44"},
                      {&g.pf_f16_sw_24, "pf_gemm_f16_swiglu_24"},
@@ -392,10 +393,8 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_f16_part_12k, "pf_gemm_f16_part_12k"},
                      {&g.pf_f16_part_44, "pf_gemm_f16_part_44"},
                      {&g.pf_f16_part_44k, "pf_gemm_f16_part_44k"},
-                     {&g.pf_rows_qkv_rope[0][0], "pf_rows_qkv_rope_1"},
-                     {&g.pf_rows_qkv_rope[0][1], "pf_rows_qkv_rope_q8_1"},
-                     {&g.pf_rows_qkv_rope[1][0], "pf_rows_qkv_rope_2"},
-                     {&g.pf_rows_qkv_rope[1][1], "pf_rows_qkv_rope_q8_2"},
+                     {&g.pf_rows_qkv_rope[0], "pf_rows_qkv_rope"},
+                     {&g.pf_rows_qkv_rope[1], "pf_rows_qkv_rope_q8"},
                      {&g.pf_rows_qkv[0][0], "pf_rows_qkv_11"},
                      {&g.pf_rows_qkv[0][1], "pf_rows_qkv_q8_11"},
                      {&g.pf_rows_qkv[1][0], "pf_rows_qkv_12"},
@@ -483,11 +482,16 @@ void q8gemv_shutdown(void) {
   }
   if (g.pf_module) (void)hipModuleUnload(g.pf_module);
   g.pf_module = nullptr;
-  g.pf_embed = g.pf_norm = g.pf_gemm = g.pf_gemm_res = g.pf_gemm_m32 = g.pf_gemm_res_m32 =
-      g.pf_gemm_swiglu = g.pf_rope = g.pf_rope_table = g.pf_attn = g.pf_attn_merge = g.pf_set_pos = nullptr;
+  g.pf_embed = g.pf_norm = g.pf_gemm_qkv = g.pf_gemm_res = g.pf_gemm_qkv_m32 = g.pf_gemm_res_m32 =
+      g.pf_gemm_swiglu = g.pf_rope = g.pf_attn = g.pf_attn_merge = g.pf_set_pos = nullptr;
   g.pf_gemm_part = g.pf_gemm_part_m32 = g.pf_res_reduce = g.pf_res_reduce_norm = nullptr;
-  g.pf_f16_44 = g.pf_f16_24 = g.pf_f16_22 = g.pf_f16_sw_46w = g.pf_f16_sw_44 = g.pf_f16_sw_24 =
-      g.pf_f16_sw_22 = nullptr;
+  g.pf_f16_qkv_44 = g.pf_f16_qkv_24 = g.pf_f16_qkv_22p = g.pf_f16_sw_46w =
+      g.pf_f16_sw_44 = g.pf_f16_sw_24 = g.pf_f16_sw_22 = nullptr;
+  std::memset(g.pf_rows_qkv_rope, 0, sizeof(g.pf_rows_qkv_rope));
+  std::memset(g.pf_rows_qkv, 0, sizeof(g.pf_rows_qkv));
+  std::memset(g.pf_rows_gu, 0, sizeof(g.pf_rows_gu));
+  std::memset(g.pf_rows_o, 0, sizeof(g.pf_rows_o));
+  std::memset(g.pf_rows_dn, 0, sizeof(g.pf_rows_dn));
   g.pf_f16_res_22 = g.pf_f16_res_22k = g.pf_f16_res_12k = g.pf_f16_part_22 = g.pf_f16_part_22k =
       g.pf_f16_part_12k = g.pf_f16_part_44 = g.pf_f16_part_44k = g.pf_expand = nullptr;
   g.vocab = g.vocab_finalize = g.argmax = g.ws_reset = g.copy = nullptr;
@@ -1520,6 +1524,13 @@ int launch_body(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
 
 // ---- batched prompt ingestion ----
 
+// What the q/k/v products write (layout shared with prefill_kernels.hip).
+struct QkvOut {
+  void *q, *k, *v, *q_roped, *k_cache, *v_cache;
+  const void *qn_w, *kn_w, *rope;
+  int start;
+};
+
 // Argument block of pf_gemm_q8* (layout shared with prefill_kernels.hip).
 struct GemmArgs {
   const void* x;
@@ -1530,23 +1541,10 @@ struct GemmArgs {
   int n_tiles;
   int ldx, ldy, ldr;
   int up_row;
-  const void* w_seg[2];  // further products with the same x (see prefill_kernels.hip)
-  void* y_seg[2];
-  int ldy_seg[2];
-  int seg_tile[2];
+  const void *wk, *wv;  // q/k/v: the further weights
+  QkvOut qkv;
   float* part;  // split-K partial sums (pf_gemm_q8_part*)
   int splits;
-};
-
-// A second and third product in the same launch: output rows n_out of w
-// / y first, then n2 rows of w2 / y2, then n3 rows of w3 / y3.
-struct GemmMore {
-  const void* w2;
-  void* y2;
-  int ldy2, n2;
-  const void* w3;
-  void* y3;
-  int ldy3, n3;
 };
 
 // Workspace regions, f16 elements per token: h, h1 (residual), xn
@@ -1630,24 +1628,10 @@ size_t pf_workspace_bytes(int32_t n) {
 // fewer than 2 workgroups per CU.
 int launch_gemm(hipFunction_t fn, hipFunction_t fn_m32, const void* x, int ldx, const void* wl,
                 int K, int n_out, int tile_cols, void* y, int ldy, const void* r, int ldr,
-                int up_row, int M, hipStream_t st, const GemmMore* more = nullptr,
-                float* part = nullptr, int splits = 1) {
-  GemmArgs a{x, wl, y, r, M, K, n_out / tile_cols, ldx, ldy, ldr, up_row,
-             {nullptr, nullptr}, {nullptr, nullptr}, {0, 0}, {0, 0}, part, splits};
-  a.seg_tile[0] = a.seg_tile[1] = a.n_tiles;
-  if (more) {
-    if (more->n2 % tile_cols != 0 || more->n3 % tile_cols != 0)
-      return fail(Q8_ERR_BAD_SHAPE, "prefill GEMM segments N=%d, %d", more->n2, more->n3);
-    a.w_seg[0] = more->w2;
-    a.y_seg[0] = more->y2;
-    a.ldy_seg[0] = more->ldy2;
-    a.w_seg[1] = more->w3;
-    a.y_seg[1] = more->y3;
-    a.ldy_seg[1] = more->ldy3;
-    a.seg_tile[0] = a.n_tiles;
-    a.seg_tile[1] = a.n_tiles + more->n2 / tile_cols;
-    a.n_tiles = a.seg_tile[1] + more->n3 / tile_cols;
-  }
+                int up_row, int M, hipStream_t st, float* part = nullptr, int splits = 1,
+                const void* wk = nullptr, const void* wv = nullptr, const QkvOut* qkv = nullptr) {
+  GemmArgs a{x, wl, y, r, M, K, n_out / tile_cols, ldx, ldy, ldr, up_row, wk, wv,
+             qkv ? *qkv : QkvOut{}, part, splits};
   // the kernel maps workgroups to n tiles in groups of 8 (one per XCD)
   if (n_out % tile_cols != 0 || a.n_tiles % 8 != 0 || K % 256 != 0)
     return fail(Q8_ERR_BAD_SHAPE, "prefill GEMM shape N=%d K=%d", n_out, K);
@@ -1678,9 +1662,7 @@ struct GemmF16Args {
   int n_tiles;
   int ldx, ldy, ldr;
   int splits;
-  void* y_seg[2];  // output columns from seg_col[0] / seg_col[1] on
-  int ldy_seg[2];
-  int seg_col[2];
+  QkvOut qkv;
 };
 
 // The f16 layer matrices (qwen3_weights.prefill_f16), f16 elements per
@@ -1710,8 +1692,7 @@ struct F16Tile {
 int launch_gemm_f16(std::initializer_list<F16Tile> tiles, const void* x, int ldx, const void* wm,
                     int K, int n_w, void* y, int ldy, const void* r, int ldr, int M,
                     hipStream_t st, float* part = nullptr, int splits = 1,
-                    const int (*seg_col)[2] = nullptr, void* const (*y_seg)[2] = nullptr,
-                    const int (*ldy_seg)[2] = nullptr) {
+                    const QkvOut* qkv = nullptr) {
   auto grid_of = [&](const F16Tile& t) {
     return ((int64_t)M + t.bm - 1) / t.bm * (n_w / t.bn) * splits;
   };
@@ -1730,17 +1711,7 @@ int launch_gemm_f16(std::initializer_list<F16Tile> tiles, const void* x, int ldx
   if (n_w % (8 * bn) != 0 || splits < 1 || K % (pick->ks * splits) != 0)
     return fail(Q8_ERR_BAD_SHAPE, "prefill f16 GEMM shape N=%d K=%d splits=%d", n_w, K, splits);
   GemmF16Args a{x, wm, y, r, part, M, K, n_w / bn, ldx, ldy, ldr, splits,
-                {nullptr, nullptr}, {0, 0}, {n_w, n_w}};
-  if (seg_col) {
-    if ((*seg_col)[0] % bn != 0 || (*seg_col)[1] % bn != 0)
-      return fail(Q8_ERR_BAD_SHAPE, "prefill f16 GEMM segments at %d, %d", (*seg_col)[0],
-                  (*seg_col)[1]);
-    for (int i = 0; i < 2; ++i) {
-      a.seg_col[i] = (*seg_col)[i];
-      a.y_seg[i] = (*y_seg)[i];
-      a.ldy_seg[i] = (*ldy_seg)[i];
-    }
-  }
+                qkv ? *qkv : QkvOut{}};
   const int64_t grid = grid_of(*pick);
   if (grid > 0x7fffffff) return fail(Q8_ERR_BAD_SHAPE, "prefill GEMM grid too large");
   void* args[] = {&a};
@@ -1804,7 +1775,7 @@ int launch_gemm_res(const void* x, int ldx, const void* wl, int K, void* y, cons
                                   x, ldx, wf16, K, kN, nullptr, kN, nullptr, 0, M, st,
                                   static_cast<float*>(part), splits)
                 : launch_gemm(g.pf_gemm_part, g.pf_gemm_part_m32, x, ldx, wl, K, kN, 64, nullptr,
-                              kN, nullptr, 0, 0, M, st, nullptr, static_cast<float*>(part),
+                              kN, nullptr, 0, 0, M, st, static_cast<float*>(part),
                               splits);
   if (rc) return rc;
   const void* pp = part;
@@ -1840,14 +1811,12 @@ struct RowsResArgs {
   int M;
 };
 
-// Most tokens the row products serve: all of a layer's products, and q/k/v
-// with RoPE alone.  At 128 tokens a layer takes 39.9 us with them and 50.6
-// with the tiled GEMMs, at 160 tokens (where a workgroup's token rows are
-// normalised by twice as many workgroups as the device has CUs) 60 and 57; the
-// q/k/v one alone pays up to 256 tokens (57.0 -> 53.7 us; 300 tokens 69.5 ->
-// 72.6).
+// Most tokens the row products serve.  At 128 tokens a layer takes 39.9 us with
+// them and 50.6 with the tiled GEMMs, at 160 tokens (where a workgroup's token
+// rows are normalised by twice as many workgroups as the device has CUs) 60 and
+// 57; the q/k/v one alone 54.0 at 160 tokens, against 50.9 with a separate norm
+// and the tiled one that ends in RoPE.
 constexpr int32_t kPfRowsMax = 128;
-constexpr int32_t kPfRowsQkvMax = 256;
 
 int launch_rows(hipFunction_t fn, int n, int tokens, int n_tiles, int threads, void* block,
                 hipStream_t st) {
@@ -1875,13 +1844,12 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
   void* vc = mb(v_cache) + (int64_t)layer * max_seq * kKvRow * 2;
   void *h = ws[0], *h1 = ws[1], *xn = ws[2], *q = ws[3], *k = ws[4], *v = ws[5], *qr = ws[6],
        *attn = ws[7], *act = ws[8], *fnx = ws[9], *part = ws[10], *rope = ws[kPfRopeRegion];
-  const uint32_t norm_grid = (uint32_t)((n + 15) / 16);
   int rc;
   // f16 layer matrices when the caller made them, else the Q8_0 stacks
   const uint8_t* f16l =
       w->prefill_f16 ? cb(w->prefill_f16) + (int64_t)layer * kPfF16Layer * 2 : nullptr;
   const int q8 = f16l ? 0 : 1;
-  const bool rows = n <= kPfRowsMax, rows_qkv = n <= kPfRowsQkvMax;
+  const bool rows = n <= kPfRowsMax;
   const void* wq = f16l ? (const void*)(f16l + kPfF16Qkv * 2) : cb(w->wq) + layer * bpl_q;
   const void* wk = cb(w->wk) + layer * bpl_kv;
   const void* wv = cb(w->wv) + layer * bpl_kv;
@@ -1892,43 +1860,43 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
     RowsNormArgs a{h, an, {wq, wk, wv}, xn, {q, k, v}, rope_ready ? nullptr : rope, n, p0};
     const int i = n <= 16 ? 0 : 1;
     if ((rc = launch_rows(g.pf_rows_qkv[i][q8], n, 16, 256 >> i, 512, &a, st))) return rc;
-  } else if (rows_qkv) {
+  } else if (rows) {
     // a whole head a workgroup, so RoPE and the cache writes fit behind it:
     // 32 workgroups per token tile, enough from about 65 tokens (64 tokens
     // 44.1 against 44.9 us a layer, 96 tokens 46.9 against 46.2)
     RowsQkvArgs a{h, an, {wq, wk, wv}, xn, q, k, v, qr, kc, vc, qn, kn, rope, n, p0,
                   rope_ready ? 1 : 0};
-    const int i = n <= kPfRowsMax ? 0 : 1;
-    if ((rc = launch_rows(g.pf_rows_qkv_rope[i][q8], n, 16 << i, 32, 512, &a, st))) return rc;
+    if ((rc = launch_rows(g.pf_rows_qkv_rope[q8], n, 16, 32, 512, &a, st))) return rc;
   }
-  if (!rows_qkv && !xn_ready) {
-    void* args[] = {&h, &an, &xn, &n};
-    if ((rc = launch(g.pf_norm, norm_grid, 256, args, st))) return rc;
-  }
-  if (rows_qkv) {
-    // done above
-  } else if (f16l) {  // q, k, v as one [4096, 1024] matrix, output columns split three ways
-    const int seg_col[2] = {2048, 3072};
-    void* const y_seg[2] = {k, v};
-    const int ldy_seg[2] = {1024, 1024};
-    if ((rc = launch_gemm_f16({{g.pf_f16_44, 128, 128, 64, 2}, {g.pf_f16_24, 64, 128, 64, 2},
-                               {g.pf_f16_22, 64, 64, 128, 0}},
-                              xn, 1024, f16l + kPfF16Qkv * 2, 1024, 4096, q, 2048, nullptr, 0, n,
-                              st, nullptr, 1, &seg_col, &y_seg, &ldy_seg)))
-      return rc;
-  } else {  // q, k, v in one launch (tiles 0-31 q, 32-47 k, 48-63 v)
-    const GemmMore kv{cb(w->wk) + layer * bpl_kv, k, 1024, 1024,
-                      cb(w->wv) + layer * bpl_kv, v, 1024, 1024};
-    if ((rc = launch_gemm(g.pf_gemm, g.pf_gemm_m32, xn, 1024, cb(w->wq) + layer * bpl_q, 1024,
-                          2048, 64, q, 2048, nullptr, 0, 0, n, st, &kv)))
-      return rc;
-  }
-  if (n <= 64 || !rows_qkv) {
+  // rms_norm, with the RoPE table of the prompt's positions (the same for
+  // every layer) where it is not there yet
+  auto norm = [&](const void* in, const void* weight, void* out, bool table) {
     int start = p0;
-    if (!rope_ready && !rows_qkv) {  // the prompt positions' angles (the same for every layer)
-      void* targs[] = {&start, &rope};
-      if ((rc = launch(g.pf_rope_table, (uint32_t)n, 64, targs, st))) return rc;
-    }
+    void* args[] = {&in, &weight, &out, &n, &start, &rope};
+    const uint32_t wgs = (uint32_t)((n + 3) / 4);
+    return launch(g.pf_norm, table ? 2 * wgs : wgs, 64, args, st);
+  };
+  if (!rows) {
+    if (!xn_ready && (rc = norm(h, an, xn, !rope_ready))) return rc;
+    const QkvOut out{q, k, v, qr, kc, vc, qn, kn, rope, p0};
+    // f16: q, k, v as one [4096, 1024] matrix, a head (128 columns) a tile.
+    // Where 64-token tiles give each CU at most one workgroup (512 tokens), the
+    // eight-wave one with six stages in LDS: 300 / 512 tokens 60.4 / 63.0 us a
+    // layer against 65.1 / 65.9 (640 tokens 85.4 against 83.8)
+    if (f16l && (int64_t)(n + 63) / 64 * 32 <= g.compute_units)
+      rc = launch_gemm_f16({{g.pf_f16_qkv_22p, 64, 128, 64, 0, 512}}, xn, 1024, wq, 1024, 4096,
+                           nullptr, 0, nullptr, 0, n, st, nullptr, 1, &out);
+    else if (f16l)
+      rc = launch_gemm_f16({{g.pf_f16_qkv_44, 128, 128, 64, 2}, {g.pf_f16_qkv_24, 64, 128, 64, 0}},
+                           xn, 1024, wq, 1024, 4096, nullptr, 0, nullptr, 0, n, st, nullptr, 1,
+                           &out);
+    else
+      rc = launch_gemm(g.pf_gemm_qkv, g.pf_gemm_qkv_m32, xn, 1024, wq, 1024, 4096, 128, nullptr, 0,
+                       nullptr, 0, 0, n, st, nullptr, 1, wk, wv, &out);
+    if (rc) return rc;
+  }
+  if (n <= 64) {
+    int start = p0;
     void* args[] = {&q, &k, &v, &start, &qn, &kn, &rope, &qr, &kc, &vc};
     if ((rc = launch(g.pf_rope, (uint32_t)n, 256, args, st))) return rc;
   }
@@ -1977,8 +1945,7 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
                             f16l ? f16l + kPfF16O * 2 : nullptr)))
     return rc;
   if (!fn_done) {
-    void* args[] = {&h1, &fn, &fnx, &n};
-    if ((rc = launch(g.pf_norm, norm_grid, 256, args, st))) return rc;
+    if ((rc = norm(h1, fn, fnx, false))) return rc;
   }
   if (f16l)
     rc = launch_gemm_f16({{g.pf_f16_sw_46w, 256, 192, 64, 1, 512},
@@ -1989,7 +1956,6 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
     rc = launch_gemm(g.pf_gemm_swiglu, nullptr, fnx, 1024, cb(w->wgu) + layer * bpl_gu, 1024, 3072,
                      32, act, 3072, nullptr, 0, 3072, n, st);
   if (rc) return rc;
-  if (rows_qkv) next_norm = nullptr;  // the next layer's q/k/v product forms its norm
   return launch_gemm_res(act, 3072, cb(w->wdn) + layer * bpl_dn, 3072, h, h1, n, part, part_bytes,
                          st, next_norm, xn, next_xn_ready, f16l ? f16l + kPfF16Dn * 2 : nullptr);
 }

@@ -1,5 +1,6 @@
-"""GPU tests of the prompt layer's row products (prefill_rows.h: all products up
-to 128 tokens, q/k/v with RoPE up to 256).
+"""GPU tests of the prompt layer's row products (prefill_rows.h, up to 128
+tokens) and of the tiled q/k/v products that end in head norms, RoPE and the
+cache writes (above).
 
 Token counts sit on the edges of their 16- and 32-token tiles and of the rules
 that pick an instance.  Each product is checked against a 64-bit product of the
@@ -12,7 +13,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_gpu_decode import fill_cache_layer
+from test_gpu_decode import f64, fill_cache_layer, rope_tol
 
 pytestmark = pytest.mark.gpu
 
@@ -100,6 +101,38 @@ def test_row_products_match_f64_and_both_weight_forms_agree(gpu, D, dmodel, w64,
     finally:
         dmodel.use_prefill_matrices(True)
         sess.free()
+
+
+@pytest.mark.parametrize("n", [1, 17, 65, 129, 257, 511, 512, 513, 1030, 1930])
+def test_head_norms_rope_and_cache(O, gpu, D, dmodel, model_host, n):
+    """q_roped, the K slots and the V slots against the oracle's head norm and
+    RoPE of the GPU's own q, k and v (2 ulp plus one ulp of the head's largest
+    input), tokens at the tile edges; both weight forms the same bits."""
+    p0 = 9
+    h_in = (1.5 * np.random.default_rng(4300 + n).standard_normal((n, 1024))).astype(np.float16)
+    sess = D.DecodeSession(dmodel, p0 + n + 1)
+    res = []
+    try:
+        for f16 in (True, False):
+            print(f"q/k/v epilogue n {n} f16 {f16}", flush=True)
+            dmodel.use_prefill_matrices(f16)
+            g = sess.prefill_layer(LAYER, h_in, p0, True)
+            res.append((g["q_roped"], g["q"], g["k"], g["v"],
+                        *sess.cache_rows(LAYER, 0, p0 + n + 1)))
+    finally:
+        dmodel.use_prefill_matrices(True)
+        sess.free()
+    for a, b in zip(*res):
+        assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
+    q_roped, q, k, v, k_rows, v_rows = res[0]
+    assert np.array_equal(v_rows[p0:p0 + n].view(np.uint16), v.view(np.uint16))
+    for rows in (k_rows, v_rows):
+        assert not rows[:p0].any() and not rows[p0 + n:].any()
+    for i in sorted({t for t in (0, 1, 15, 16, 63, 64, 127, 128, n // 2, n - 2, n - 1) if 0 <= t < n}):
+        for x, w, got in ((q, model_host.q_norm, q_roped[i]), (k, model_host.k_norm, k_rows[p0 + i])):
+            normed = O.head_rmsnorm(x[i], w[LAYER])
+            want = O.rope(normed, p0 + i)
+            assert (np.abs(f64(got) - f64(want)) <= rope_tol(O, normed, want)).all(), i
 
 
 @pytest.mark.parametrize("n", [16, 100, 200])
