@@ -918,10 +918,10 @@ extern "C" __global__ __launch_bounds__(64) void pf_rmsnorm(const uint16_t* __re
   }
 }
 
-extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_qkv(GemmArgs A) {
+extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8(GemmArgs A) {
   gemm_q8<kEpiQkv, 64>(A);
 }
-extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_qkv_m32(GemmArgs A) {
+extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_m32(GemmArgs A) {
   gemm_q8<kEpiQkv, 32>(A);
 }
 extern "C" __global__ __launch_bounds__(256) void pf_gemm_q8_res(GemmArgs A) {

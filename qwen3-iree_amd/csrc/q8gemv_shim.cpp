@@ -365,9 +365,9 @@ int q8gemv_init(const char* code_object_path) {
           const char* name;
         } names[] = {{&g.pf_embed, "pf_embed"},
                      {&g.pf_norm, "pf_rmsnorm"},
-                     {&g.pf_gemm_qkv, "pf_gemm_q8_qkv"},
+                     {&g.pf_gemm_qkv, "pf_gemm_q8"},
                      {&g.pf_gemm_res, "pf_gemm_q8_res"},
-                     {&g.pf_gemm_qkv_m32, "pf_gemm_q8_qkv_m32"},
+                     {&g.pf_gemm_qkv_m32, "pf_gemm_q8_m32"},
                      {&g.pf_gemm_res_m32, "pf_gemm_q8_res_m32"},
                      {&g.pf_gemm_swiglu, "pf_gemm_q8_swiglu"},
                      {&g.pf_rope, "pf_qk_rope_cache"},
