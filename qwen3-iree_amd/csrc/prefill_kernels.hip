@@ -1169,16 +1169,56 @@ extern "C" __global__ __launch_bounds__(256) void pf_qk_rope_cache(
 // (1 MiB at 2048 positions) instead of all eight.  A query
 // block with one split writes its output directly; otherwise each split
 // leaves its partial in its slot of `part` and pf_attn_merge, launched next,
-// combines them.
+// combines them.  Workgroups from attn_wgs on touch weights instead.
 
 // How far (base-2 units) a block's maximum score may exceed the reference
 // maximum before the reference moves (the weights' range is [0, 2^kMaxLag]).
 constexpr float kMaxLag = 8.0f;
 
+// Weights the layer's later launches read, brought into the caches by further
+// workgroups of the attention launch, which leaves HBM idle: per matrix its
+// tiles, each into the L2 of the XCD that will multiply it (tile n on XCD n mod
+// 8).  The 28 layers' 880 MB do not stay in the memory-side cache, and the
+// products after the attention wait for HBM: 1021 tokens took 108 us a layer
+// inside a prompt against 92 for one layer over and over.  Whole prompts of
+// 24 / 64 / 128 / 300 / 512 / 1021 tokens: 946 / 1087 / 1234 / 1942 / 1974 /
+// 3098 -> 928 / 1045 / 1177 / 1729 / 1788 / 2735 us.  (Half of the weights from
+// the RoPE launch, for up to 64 tokens: 925 and 1049.)
+constexpr int kPfTouchMats = 7;
+struct PfTouch {
+  const uint8_t* base[kPfTouchMats];
+  int tile_bytes[kPfTouchMats];  // a multiple of 128
+  int tiles[kPfTouchMats];       // a multiple of 8
+};
+
+// Workgroup `rank` of `ranks` on this XCD (workgroup mod 8) touches its share
+// of the lines of the XCD's tiles: one dword of each 128-byte line, 64 lines
+// per load, into the wave's never-read part of `sink`.
+__device__ __forceinline__ void touch_weights(const PfTouch& T, int xcd, int rank, int ranks,
+                                              uint8_t* sink) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < kPfTouchMats; ++i) {
+    if (T.tiles[i] == 0) continue;
+    const int tile_lines = T.tile_bytes[i] / 128;
+    const int lines = T.tiles[i] / 8 * tile_lines;  // this XCD's
+    for (int l0 = 64 * (4 * rank + wave); l0 < lines; l0 += 256 * ranks) {
+      const int l = l0 + lane < lines ? l0 + lane : lines - 1;
+      const int tile = l / tile_lines;
+      const uint8_t* p = T.base[i] + (size_t)(8 * tile + xcd) * T.tile_bytes[i] +
+                         128 * (l - tile * tile_lines);
+      __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)p, (LDS_AS void*)(sink + 256 * wave),
+                                       4, 0, 0);
+    }
+  }
+  wait_vm<0>();  // the copies land before the workgroup's LDS is given away
+}
+
 extern "C" __global__ __launch_bounds__(256) void pf_attention(
     const uint16_t* __restrict__ q_roped, const uint16_t* __restrict__ k_cache,
     const uint16_t* __restrict__ v_cache, int n, int start, int chunk_local, int split_blocks,
-    float* __restrict__ part, uint16_t* __restrict__ out) {
+    float* __restrict__ part, uint16_t* __restrict__ out, int attn_wgs, PfTouch touch) {
   // K and V tiles of two blocks: separate arrays so the compiler sees that
   // reading one buffer does not wait for the copies into the other.  (Three,
   // two blocks copied ahead, 48 KiB of LDS against 32: 4.83 against 4.80 ms
@@ -1186,6 +1226,11 @@ extern "C" __global__ __launch_bounds__(256) void pf_attention(
   __shared__ __attribute__((aligned(1024))) uint8_t kt0[8192], kt1[8192];
   __shared__ __attribute__((aligned(1024))) uint8_t vt0[8192], vt1[8192];
   const int g = blockIdx.x & 7;
+  if ((int)blockIdx.x >= attn_wgs) {
+    touch_weights(touch, g, ((int)blockIdx.x - attn_wgs) >> 3, ((int)launch_wgs() - attn_wgs) >> 3,
+                  kt0);
+    return;
+  }
   const int pair = blockIdx.x >> 3;
   const int t = threadIdx.x;
   const int wave = t >> 6;

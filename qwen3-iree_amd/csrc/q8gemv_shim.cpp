@@ -1818,6 +1818,54 @@ struct RowsResArgs {
 // and the tiled one that ends in RoPE.
 constexpr int32_t kPfRowsMax = 128;
 
+// Weights the attention launch's further workgroups bring into the caches
+// (layout shared with prefill_kernels.hip).
+constexpr int kPfTouchMats = 7;
+struct PfTouch {
+  const void* base[kPfTouchMats];
+  int tile_bytes[kPfTouchMats];
+  int tiles[kPfTouchMats];
+};
+
+// attn_o, gate/up, ffn_down and, above 128 tokens (where the next layer's q/k/v
+// product is long enough away for nothing to be evicted: 128 tokens 1177 us a
+// prompt without, 1189 with; 300 tokens 1765 and 1729), the next layer's q, k
+// and v, in the tiles their products will use for n tokens.  A tile that is
+// taken to be another only lands in another XCD's L2.
+PfTouch touch_plan(const qwen3_weights* w, int layer, int32_t n) {
+  PfTouch t{};
+  int mats = 0;
+  auto add = [&](const uint8_t* base, int row_bytes, int rows, int tile_rows) {
+    t.base[mats] = base;
+    t.tile_bytes[mats] = row_bytes * tile_rows;
+    t.tiles[mats++] = rows / tile_rows;
+  };
+  const bool rows = n <= kPfRowsMax, next = !rows && layer + 1 < kLayers;
+  const int rows_gu = n <= 32 ? 32 : (n <= 64 ? 64 : 96);
+  if (w->prefill_f16) {
+    const uint8_t* f = cb(w->prefill_f16) + (int64_t)layer * kPfF16Layer * 2;
+    const int res = rows ? 16 : ((n + 127) / 128 * 16 >= g.compute_units ? 128 : 64);
+    add(f + kPfF16O * 2, 2 * 2048, 1024, res);
+    add(f + kPfF16Gu * 2, 2 * 1024, 6144, rows ? rows_gu : (n > 1792 ? 192 : (n > 640 ? 128 : 64)));
+    add(f + kPfF16Dn * 2, 2 * 3072, 1024, res);
+    if (next) add(f + (kPfF16Layer + kPfF16Qkv) * 2, 2 * 1024, 4096, 128);
+  } else {
+    const int64_t l = layer, r1 = 1088, r2 = 2176, r3 = 3264;  // row bytes of K = 1024, 2048, 3072
+    const uint8_t* gu = cb(w->wgu) + l * 6144 * r1;
+    const int res = rows ? 16 : 64, half = rows ? rows_gu / 2 : 32;
+    add(cb(w->wo) + l * 1024 * r2, (int)r2, 1024, res);
+    add(gu, (int)r1, 3072, half);
+    add(gu + 3072 * r1, (int)r1, 3072, half);
+    add(cb(w->wdn) + l * 1024 * r3, (int)r3, 1024, res);
+    if (next) {
+      add(cb(w->wq) + (l + 1) * 2048 * r1, (int)r1, 2048, 128);
+      add(cb(w->wk) + (l + 1) * 1024 * r1, (int)r1, 1024, 128);
+      add(cb(w->wv) + (l + 1) * 1024 * r1, (int)r1, 1024, 128);
+    }
+  }
+  return t;
+}
+
 int launch_rows(hipFunction_t fn, int n, int tokens, int n_tiles, int threads, void* block,
                 hipStream_t st) {
   void* args[] = {block};
@@ -1828,11 +1876,14 @@ int launch_rows(hipFunction_t fn, int n, int tokens, int n_tiles, int threads, v
 // attn_norm of this layer) (written by the previous layer's last reduce).
 // next_norm (the next layer's attn_norm, or null): if ffn_down's reduce can
 // also form the next layer's xn it does so and *next_xn_ready becomes true.
+// whole_prompt: the other layers run before and after, so the attention launch
+// also brings the following weights into the caches (a layer by itself may find
+// them there: 512 tokens 62.4 us a layer over and over, 64.1 with).
 int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void* v_cache,
                          int64_t max_seq, int32_t n, int32_t p0, int chunk_local,
                          void* const (&ws)[kPfRegions], hipStream_t st, bool xn_ready = false,
                          const void* next_norm = nullptr, bool* next_xn_ready = nullptr,
-                         bool rope_ready = false) {
+                         bool rope_ready = false, bool whole_prompt = false) {
   const int64_t bpl_q = 2048LL * 1024 / 32 * 34, bpl_kv = 1024LL * 1024 / 32 * 34;
   const int64_t bpl_o = 1024LL * 2048 / 32 * 34, bpl_gu = 6144LL * 1024 / 32 * 34;
   const int64_t bpl_dn = 1024LL * 3072 / 32 * 34;
@@ -1907,9 +1958,12 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
     const int64_t pairs = pf_pairs_total(G, sb);
     if (pairs > pf_attn_pair_cap(n))
       return fail(Q8_ERR_BAD_SHAPE, "attention splits exceed the workspace");  // not reached
-    void* args[] = {&qr, &kc, &vc, &nn, &start, &cl, &sb, &part, &attn};
+    PfTouch touch = whole_prompt ? touch_plan(w, layer, n) : PfTouch{};
+    const uint32_t touch_wgs = !whole_prompt ? 0 : (n <= 64 ? 256 : 128);
+    int attn_wgs = (int)(8 * pairs);
+    void* args[] = {&qr, &kc, &vc, &nn, &start, &cl, &sb, &part, &attn, &attn_wgs, &touch};
     // 1-D grids, kv head = workgroup mod 8: one head per XCD
-    if ((rc = launch(g.pf_attn, (uint32_t)(8 * pairs), 256, args, st))) return rc;
+    if ((rc = launch(g.pf_attn, (uint32_t)attn_wgs + touch_wgs, 256, args, st))) return rc;
     if (pairs > G.nqb) {  // some query block has several splits
       void* margs[] = {&part, &nn, &start, &cl, &sb, &attn};
       if ((rc = launch(g.pf_attn_merge, (uint32_t)(32 * G.nqb), 256, margs, st))) return rc;
@@ -2476,7 +2530,7 @@ int qwen3_prefill_batched(const qwen3_weights* w, void* k_cache, void* v_cache, 
   for (int l = 0; l < kLayers; ++l) {
     const void* next_norm = l + 1 < kLayers ? cb(w->attn_norm) + (l + 1) * 2048 : nullptr;
     if ((rc = launch_prefill_layer(w, l, k_cache, v_cache, max_seq, n_prompt, p0, chunk_local, ws,
-                                   st, xn_ready, next_norm, &xn_ready, l > 0)))
+                                   st, xn_ready, next_norm, &xn_ready, l > 0, true)))
       return rc;
   }
   {
