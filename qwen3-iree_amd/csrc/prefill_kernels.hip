@@ -675,8 +675,9 @@ __device__ __forceinline__ void pf_static_for(F&& f) {
   }
 }
 
-template <int EPI, int STAGES, int MS, int NS, int NBUF, int WM, int WN>
+template <int EPI, int STAGES, int MS, int NS, int NBUF, int WM, int WN, int CHAINS = 1>
 __device__ __forceinline__ void gemm_pipe(const GemmF16Args& A) {
+  static_assert(CHAINS == 1 || (CHAINS == 2 && STAGES % 2 == 0), "K ranges");
   static_assert(NBUF >= 3 && NBUF <= 6, "buffers");
   constexpr int KS = 64;
   constexpr int kWaves = WM * WN;
@@ -743,6 +744,7 @@ __device__ __forceinline__ void gemm_pipe(const GemmF16Args& A) {
   for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
     for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 first[MS][NS];  // CHAINS == 2: the first K range's sums
   f16x8 a[2][MS], b[2][NS];
   auto read = [&](const uint8_t* buf, int kb) {
 #pragma unroll
@@ -774,6 +776,15 @@ __device__ __forceinline__ void gemm_pipe(const GemmF16Args& A) {
   // NBUF - 1
   auto step = [&](auto left, int s, const uint8_t* cur, const uint8_t* next, uint8_t* refill) {
     constexpr int kLeft = decltype(left)::value;
+    if (CHAINS == 2 && s == STAGES / 2) {
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+        for (int ns = 0; ns < NS; ++ns) {
+          first[ms][ns] = acc[ms][ns];
+          acc[ms][ns] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
     wait_lds();
     read(cur, 1);
     __builtin_amdgcn_sched_barrier(0);
@@ -806,6 +817,12 @@ __device__ __forceinline__ void gemm_pipe(const GemmF16Args& A) {
          bufs[kI % NBUF], bufs[(kI + 1) % NBUF], bufs[(kI + NBUF - 1) % NBUF]);
   });
 
+  if constexpr (CHAINS == 2) {
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = first[ms][ns] + acc[ms][ns];
+  }
   gemm_f16_epilogue<EPI, MS, NS, WM, WN, kBuf>(A, acc, lds0, m0, n_tile, split);
 }
 
@@ -1031,6 +1048,29 @@ PF_GEMM_F16(pf_gemm_f16_part_12k, kEpiPartial, 1, 2, 256, 3)
 PF_GEMM_F16(pf_gemm_f16_part_44, kEpiPartial, 4, 4, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_part_44k, kEpiPartial, 4, 4, 128, 2)
 #undef PF_GEMM_F16
+// attn_o (32 stages of K) and ffn_down (48) with the residual in the epilogue
+// where one round of workgroups covers the tokens: 64 x 64 tiles (513 to 1024
+// tokens) or 128 x 64 over eight waves (to about 2560), instead of f32 sums to
+// memory and a reduce launch.  C chains: the K ranges the token count calls
+// for (2: the first half's sums kept aside), the bits of the split product and
+// its reduce.  Layer at 640 / 800 / 1280 / 1500 / 1800 / 2048 tokens: 85.3 /
+// 90.1 / 133.9 / 148.0 / 169.8 / 158.1 -> 77.7 / 82.7 / 112.6 / 125.2 / 145.7 /
+// 147.8 us; at 512 tokens the split product stays (64.0 against 69.2), at 4096
+// the 128 x 128 one (355 against 370).
+#define PF_GEMM_RES_P(suffix, MS, WM, WN, C)                                                  \
+  extern "C" __global__ __launch_bounds__(64 * WM * WN) void pf_gemm_f16_res_o_##suffix(      \
+      GemmF16Args A) {                                                                        \
+    gemm_pipe<kEpiResidual, 32, MS, 2, 6, WM, WN, C>(A);                                      \
+  }                                                                                           \
+  extern "C" __global__ __launch_bounds__(64 * WM * WN) void pf_gemm_f16_res_dn_##suffix(     \
+      GemmF16Args A) {                                                                        \
+    gemm_pipe<kEpiResidual, 48, MS, 2, 6, WM, WN, C>(A);                                      \
+  }
+PF_GEMM_RES_P(p1, 2, 2, 2, 1)
+PF_GEMM_RES_P(p2, 2, 2, 2, 2)
+PF_GEMM_RES_P(w1, 2, 4, 2, 1)
+PF_GEMM_RES_P(w2, 2, 4, 2, 2)
+#undef PF_GEMM_RES_P
 
 // Per-head rms_norm (q_norm / k_norm, qwen3_full.mlir:648-702) and RoPE
 // (:324-454) of one head vector: lane owns dims 2 lane, 2 lane + 1 (xw, an

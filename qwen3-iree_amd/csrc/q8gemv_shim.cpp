@@ -131,6 +131,8 @@ struct State {
                 pf_f16_res_22 = nullptr, pf_f16_res_22k = nullptr, pf_f16_res_12k = nullptr,
                 pf_f16_part_22 = nullptr, pf_f16_part_22k = nullptr, pf_f16_part_12k = nullptr,
                 pf_f16_part_44 = nullptr, pf_f16_part_44k = nullptr, pf_expand = nullptr;
+  // [64 x 64, 128 x 64 tiles][attn_o, ffn_down][K ranges - 1]
+  hipFunction_t pf_f16_res_pipe[2][2][2] = {};
   // the row products (prefill_rows.h): [instance, fewest tokens first][0: f16
   // weights, 1: Q8_0]
   hipFunction_t pf_rows_qkv_rope[2] = {}, pf_rows_qkv[2][2] = {}, pf_rows_gu[4][2] = {},
@@ -388,6 +390,14 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_f16_res_22, "pf_gemm_f16_res_22"},
                      {&g.pf_f16_res_22k, "pf_gemm_f16_res_22k"},
                      {&g.pf_f16_res_12k, "pf_gemm_f16_res_12k"},
+                     {&g.pf_f16_res_pipe[0][0][0], "pf_gemm_f16_res_o_p1"},
+                     {&g.pf_f16_res_pipe[0][0][1], "pf_gemm_f16_res_o_p2"},
+                     {&g.pf_f16_res_pipe[0][1][0], "pf_gemm_f16_res_dn_p1"},
+                     {&g.pf_f16_res_pipe[0][1][1], "pf_gemm_f16_res_dn_p2"},
+                     {&g.pf_f16_res_pipe[1][0][0], "pf_gemm_f16_res_o_w1"},
+                     {&g.pf_f16_res_pipe[1][0][1], "pf_gemm_f16_res_o_w2"},
+                     {&g.pf_f16_res_pipe[1][1][0], "pf_gemm_f16_res_dn_w1"},
+                     {&g.pf_f16_res_pipe[1][1][1], "pf_gemm_f16_res_dn_w2"},
                      {&g.pf_f16_part_22, "pf_gemm_f16_part_22"},
                      {&g.pf_f16_part_22k, "pf_gemm_f16_part_22k"},
                      {&g.pf_f16_part_12k, "pf_gemm_f16_part_12k"},
@@ -487,6 +497,7 @@ void q8gemv_shutdown(void) {
   g.pf_gemm_part = g.pf_gemm_part_m32 = g.pf_res_reduce = g.pf_res_reduce_norm = nullptr;
   g.pf_f16_qkv_44 = g.pf_f16_qkv_24 = g.pf_f16_qkv_22p = g.pf_f16_sw_46w =
       g.pf_f16_sw_44 = g.pf_f16_sw_24 = g.pf_f16_sw_22 = nullptr;
+  std::memset(g.pf_f16_res_pipe, 0, sizeof(g.pf_f16_res_pipe));
   std::memset(g.pf_rows_qkv_rope, 0, sizeof(g.pf_rows_qkv_rope));
   std::memset(g.pf_rows_qkv, 0, sizeof(g.pf_rows_qkv));
   std::memset(g.pf_rows_gu, 0, sizeof(g.pf_rows_gu));
@@ -1756,6 +1767,21 @@ int launch_gemm_res(const void* x, int ldx, const void* wl, int K, void* y, cons
     }
     if ((size_t)splits * M * kN * 4 > part_bytes) splits = 1;
   }
+  // One round of workgroups that finish their outputs themselves, where there
+  // is such a grid (figures beside the kernels; whole prompts of 640 / 1021
+  // tokens with other weights each time 2527 / 2922 -> 2336 / 2761 us, ffn_down
+  // alone 2416 / 2823); a norm that follows is the caller's.
+  if (wf16 && splits <= 2 && g.pf_tile_rows.load(std::memory_order_relaxed) == 0) {
+    const int64_t wgs64 = ((int64_t)M + 63) / 64 * (kN / 64);
+    const int64_t wgs128n = ((int64_t)M + 127) / 128 * (kN / 64);
+    const int k = K == 2048 ? 0 : 1;
+    if (M > 512 && wgs64 <= g.compute_units)
+      return launch_gemm_f16({{g.pf_f16_res_pipe[0][k][splits - 1], 64, 64, 64, 0}}, x, ldx, wf16,
+                             K, kN, y, kN, r, kN, M, st);
+    if (M > 512 && 4 * wgs128n <= 5LL * g.compute_units)
+      return launch_gemm_f16({{g.pf_f16_res_pipe[1][k][splits - 1], 128, 64, 64, 0, 512}}, x, ldx,
+                             wf16, K, kN, y, kN, r, kN, M, st);
+  }
   // with a norm to form, even an unsplit K goes through the f32 sums and the
   // reduce (which adds the residual exactly as the GEMM epilogue would):
   // 1024 tokens 4.24 -> 4.13 ms, 2048 tokens 7.69 -> 7.61 ms
@@ -1844,7 +1870,7 @@ PfTouch touch_plan(const qwen3_weights* w, int layer, int32_t n) {
   const int rows_gu = n <= 32 ? 32 : (n <= 64 ? 64 : 96);
   if (w->prefill_f16) {
     const uint8_t* f = cb(w->prefill_f16) + (int64_t)layer * kPfF16Layer * 2;
-    const int res = rows ? 16 : ((n + 127) / 128 * 16 >= g.compute_units ? 128 : 64);
+    const int res = rows ? 16 : (n > 2560 ? 128 : 64);
     add(f + kPfF16O * 2, 2 * 2048, 1024, res);
     add(f + kPfF16Gu * 2, 2 * 1024, 6144, rows ? rows_gu : (n > 1792 ? 192 : (n > 640 ? 128 : 64)));
     add(f + kPfF16Dn * 2, 2 * 3072, 1024, res);

@@ -135,6 +135,30 @@ def test_head_norms_rope_and_cache(O, gpu, D, dmodel, model_host, n):
             assert (np.abs(f64(got) - f64(want)) <= rope_tol(O, normed, want)).all(), i
 
 
+@pytest.mark.parametrize("n", [513, 575, 992, 993, 1024, 1025, 1153, 1920, 1921, 2047, 2560, 2561])
+def test_unsplit_residual_products(gpu, D, dmodel, w64, n):
+    """attn_o and ffn_down around the edges of the one-round products with the
+    residual in the epilogue (513 to 2560 tokens, one K range or two): the
+    64-bit product's bound on the first and last token tiles, and the bits of
+    the Q8_0 route (split products and their reduce)."""
+    h_in = (1.5 * np.random.default_rng(4400 + n).standard_normal((n, 1024))).astype(np.float16)
+    sess = D.DecodeSession(dmodel, n)
+    res = []
+    try:
+        for f16 in (True, False):
+            print(f"residual products n {n} f16 {f16}", flush=True)
+            dmodel.use_prefill_matrices(f16)
+            res.append(sess.prefill_layer(LAYER, h_in, 0))
+    finally:
+        dmodel.use_prefill_matrices(True)
+        sess.free()
+    ga, gb = res
+    for name in ga:
+        assert np.array_equal(ga[name].view(np.uint16), gb[name].view(np.uint16)), name
+    rows = np.r_[0:130, n - 130:n]
+    check_layer({name: a[rows] for name, a in ga.items()}, h_in[rows], w64)
+
+
 @pytest.mark.parametrize("n", [16, 100, 200])
 def test_row_products_with_the_prompts_rope_table(gpu, D, dmodel, model_host, n):
     """qwen3_prefill_batched computes the RoPE table in its first layer and
