@@ -130,7 +130,7 @@ struct State {
                 pf_f16_sw_22 = nullptr,
                 pf_f16_res_22 = nullptr, pf_f16_res_22k = nullptr, pf_f16_res_12k = nullptr,
                 pf_f16_part_22 = nullptr, pf_f16_part_22k = nullptr, pf_f16_part_12k = nullptr,
-                pf_f16_part_44 = nullptr, pf_f16_part_44k = nullptr, pf_expand = nullptr;
+                pf_f16_part_44k = nullptr, pf_expand = nullptr;
   // [64 x 64, 128 x 64 tiles][attn_o, ffn_down][K ranges - 1]
   hipFunction_t pf_f16_res_pipe[2][2][2] = {};
   // the row products (prefill_rows.h): [instance, fewest tokens first][0: f16
@@ -401,7 +401,6 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_f16_part_22, "pf_gemm_f16_part_22"},
                      {&g.pf_f16_part_22k, "pf_gemm_f16_part_22k"},
                      {&g.pf_f16_part_12k, "pf_gemm_f16_part_12k"},
-                     {&g.pf_f16_part_44, "pf_gemm_f16_part_44"},
                      {&g.pf_f16_part_44k, "pf_gemm_f16_part_44k"},
                      {&g.pf_rows_qkv_rope[0], "pf_rows_qkv_rope"},
                      {&g.pf_rows_qkv_rope[1], "pf_rows_qkv_rope_q8"},
@@ -504,7 +503,7 @@ void q8gemv_shutdown(void) {
   std::memset(g.pf_rows_o, 0, sizeof(g.pf_rows_o));
   std::memset(g.pf_rows_dn, 0, sizeof(g.pf_rows_dn));
   g.pf_f16_res_22 = g.pf_f16_res_22k = g.pf_f16_res_12k = g.pf_f16_part_22 = g.pf_f16_part_22k =
-      g.pf_f16_part_12k = g.pf_f16_part_44 = g.pf_f16_part_44k = g.pf_expand = nullptr;
+      g.pf_f16_part_12k = g.pf_f16_part_44k = g.pf_expand = nullptr;
   g.vocab = g.vocab_finalize = g.argmax = g.ws_reset = g.copy = nullptr;
   g.calib_empty = g.calib_handoff = g.calib_chase = g.read = nullptr;
   g.ready = false;
@@ -1736,7 +1735,8 @@ int launch_gemm_f16(std::initializer_list<F16Tile> tiles, const void* x, int ldx
 // once but not twice (about 512-1023 tokens), K is split in two, since one
 // workgroup per CU walking all of K hides too little load latency; where
 // 128 x 128 tiles cover the CUs once in two K ranges but not in one (about
-// 2048-4095 tokens), K is split in two for those tiles.  The split
+// 2048-4095 tokens), K is split in two for those tiles (over f16 weights 513
+// to 2560 tokens instead finish in one launch, see below).  The split
 // count depends on M only, so every token tile gives the same bits.  With
 // norm_w set and K split, the reduce also writes norm_out = rms_norm(y,
 // norm_w) (pf_res_reduce_norm, the bits of a separate pf_rmsnorm) and
