@@ -645,11 +645,11 @@ constexpr int kVecWords = kAttnGroupsMax * 130;  // 2080: the largest polled vec
 // kernel arguments preloaded (508.5 / 511.4 as below): D 26 / 34 526.8 /
 // 542.6, A 28 / 36 515.1 / 524.4, C 26 / 34 515.3 / 529.5, E 12 / 20 512.2 /
 // 510.9.
-// With split groups 8 .. 15 in the code (context 1024 / 16384): A 28 / 30 / 32
-// / 34 519 / 513 / 516 / 522 and 1016 / 1011 / 1008 / 1006, so A sleeps 30 where
-// a split is one chunk and 32 where the attention takes longer (2048: 592 at 30,
-// 588 at 32); C 28 / 32 517-519, D 28 / 32 521 / 530, E 12 / 20 and the
-// cache chunk 4 / 12 within 1.
+// With split groups 8 .. 15 in the code: A 28 / 29 / 30 / 31 at context 1024
+// 522 / 516.5 / 514 / 514, 1030 560 / 560 / 560.5 / 563, 1500 572 / 570.6 / 570.4
+// / 572, 2048 594 / 592 / 590 / 590, 16384 1018 / 1015 / 1014 / 1011 (30 to
+// 1024 positions and 32 above: 565, 574, 590, 1008); C 28 / 32 517-519, D 28 /
+// 32 521 / 530, E 12 / 20 and the cache chunk 4 / 12 within 1.
 #ifndef DEC_PACE_A
 #define DEC_PACE_A 30
 #endif
@@ -871,10 +871,8 @@ void dec_step(StepParams P) {
                    step_tag(seq, layer, kPhAct));
         STAMP(layer, 10);
       }
-      if (layer + 1 < kLayers) {
-        if (n_split_chunks == 1) q8_quad_prefetch<1, kPaceA>(wsel + (layer + 1) * bpl, n, qd, la);
-        else q8_quad_prefetch<1, kPaceA + 2>(wsel + (layer + 1) * bpl, n, qd, la);
-      }
+      if (layer + 1 < kLayers)
+        q8_quad_prefetch<1, kPaceA>(wsel + (layer + 1) * bpl, n, qd, la);
     }
   } else if (wg < kCBase || wg >= kStepWgs) {
     // ================= B: attention (+ merge on split group 0) =================
