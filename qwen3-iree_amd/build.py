@@ -100,8 +100,9 @@ def build_shim() -> Path:
 # includes)
 OBJECT_SOURCES = {
     "q8gemv": ("q8gemv_kernels.hip", "q8_device.h"),
-    "decode": ("decode_kernels.hip", "decode_device.h", "q8_device.h"),
-    "prefill": ("prefill_kernels.hip", "prefill_rows.h", "prefill_split.h", "decode_device.h", "q8_device.h"),
+    "decode": ("decode_kernels.hip", "decode_device.h", "step_roles.h", "q8_device.h"),
+    "prefill": ("prefill_kernels.hip", "prefill_rows.h", "prefill_split.h", "decode_device.h",
+                "step_roles.h", "q8_device.h"),
 }
 
 

@@ -6,6 +6,7 @@
 #define QWEN3_DECODE_DEVICE_H
 
 #include "q8_device.h"
+#include "step_roles.h"
 
 namespace {
 
@@ -27,7 +28,6 @@ constexpr int kVocab = 151936;
 // merge).  Two chunks ahead with K rows straight to registers, without more
 // waves, was slower (1331 at 16384: the gathered row loads).
 constexpr int kAttnSplits = 32;
-constexpr int kAttnShortCtx = 2048;
 constexpr int kAttnWaves = 4;        // splits per workgroup, merged in LDS
 constexpr int kAttnGroups = kAttnSplits / kAttnWaves;  // partials per query head
 constexpr int kAttnGroupsMax = 2 * kAttnGroups;
@@ -325,7 +325,7 @@ __device__ __forceinline__ void rope_angles(int pos, float (&cs)[2], float (&sn)
 // log2 of the number of splits of the attention at (clamped) position pos.
 __device__ __forceinline__ int attn_splits_log2(int pos) {
   static_assert(kAttnSplits == 32, "log2");
-  return pos < kAttnShortCtx ? 5 : 6;
+  return step_long(pos) ? 6 : 5;
 }
 __device__ __forceinline__ int attn_splits(int pos) { return 1 << attn_splits_log2(pos); }
 // Its chunks of 32 positions per split (the most any split has).

@@ -356,10 +356,6 @@ extern "C" __global__ __launch_bounds__(256) void dec_scratch_clear(uint32_t* __
 // word, and every waiting workgroup gives up.
 namespace {
 
-constexpr int kStepWgs = 448;
-// The launch: 64 more workgroups (the second slot of the remaining CUs), which
-// take split groups 8 .. 15 of a context of 64 splits and end at once below.
-constexpr int kStepGrid = 512;
 constexpr int kAdBase = 0, kDCount = 192;  // A on all 256, D on the first 192
 constexpr int kBBase = 256;                // 64 attention workgroups
 constexpr int kCBase = 320;                // 128 attn_o + ffn_down workgroups
@@ -399,9 +395,11 @@ constexpr int kWRes = kWAtt + kRep * kNAtt;                // kRep x 512
 constexpr int kWAct = kWRes + kRep * kNRes;                // kRep x 1536
 constexpr int kWParity = kWAct + kRep * kNAct;
 constexpr int kWArg = 2 * kWParity;                        // 2 per workgroup
-constexpr int kWTotal = kWArg + 2 * kStepWgs;
+constexpr int kWStarted = kWArg + 2 * kStepWgs;            // 1 per extra workgroup (step_roles.h)
+constexpr int kWTotal = kWStarted + kStepExtra;
 // phases in a tag
 constexpr int kPhQKV = 0, kPhPart = 1, kPhAtt = 2, kPhRes = 3, kPhAct = 4, kPhH = 5, kPhArg = 6;
+constexpr int kPhStarted = 7;  // of layer kLayers
 
 struct StepParams {
   const uint16_t* token_embd;
@@ -574,6 +572,30 @@ struct Waiter {
   }
 };
 
+// The memory behind step_start_extra and step_may_end.
+struct ExtraIo {
+  const StepParams& P;
+  __device__ uint32_t load_seq() const {
+    return __hip_atomic_load(P.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ uint32_t load_status() const {
+    return __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ int32_t load_pos() const {
+    return __hip_atomic_load(P.pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ void put_started(int i, uint32_t seq, int32_t pos) const {
+    put_word(P.words + kWStarted + i, (uint32_t)pos, step_tag(seq, kLayers, kPhStarted));
+  }
+};
+struct EndIo {
+  const Waiter& W;
+  const uint64_t* started;
+  uint32_t tag;
+  uint32_t* vec;
+  __device__ bool wait_started() const { return W.wait(started, kStepExtra, tag, vec); }
+};
+
 // Row sums of a quad (rows q4, q4+1, q4+2, q4+3; row r's sum in lanes
 // 16(r - q4)..) published as two f16-pair words, 2 quad and 2 quad + 1, in
 // REP replicas `stride` words apart: lanes 0..REP-1 write the first word,
@@ -740,17 +762,33 @@ void dec_step(StepParams P) {
   // advances the position nor writes a token.  A thread that reads a number a
   // give-up has already advanced also sees the bit (set before the number
   // moves), so a workgroup that runs has one number in every thread.
-  const uint32_t seq = __hip_atomic_load(P.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-  const uint32_t status_in = __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t seq = 0, status_in = 0;
+  int pos_raw = 0;
+  if (wg < kStepWgs) {
+    seq = __hip_atomic_load(P.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    status_in = __hip_atomic_load(P.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    pos_raw = *P.pos;
+  } else if (t == 0) {
+    // may run after the step's end (step_roles.h): one thread reads, and says so
+    ExtraIo io{P};
+    const StepStart st = step_start_extra(io, wg - kStepWgs);
+    vec[0] = st.seq;
+    vec[1] = st.status;
+    vec[2] = (uint32_t)st.pos;
+  }
   __syncthreads();  // s_abort is 0 in every thread's view
+  if (wg >= kStepWgs) {
+    seq = vec[0];
+    status_in = vec[1];
+    pos_raw = (int)vec[2];
+  }
   if ((status_in & 2u) != 0u) s_abort = 1;
   if (P.spin_limit == 0u && wg == 0 && t == 0 && (status_in & 2u) == 0u) {
     give_up(P.status, P.seq, seq);  // the host forces a give-up
     s_abort = 1;
   }
-  const int pos_raw = *P.pos;
   const int pos_c = pos_raw < 0 ? 0 : (pos_raw >= P.max_seq ? P.max_seq - 1 : pos_raw);
-  const bool long_ctx = attn_splits(pos_c) != kAttnSplits;
+  const bool long_ctx = step_long(pos_c);
   // Workgroups start in index order: the last one of those every context needs
   // marks the launch as
   // resident (a wait that finds another number after ~1 ms knows the grid
@@ -1125,6 +1163,10 @@ void dec_step(StepParams P) {
 #endif
   // ---- workgroup 0: token, position, sequence number ----
   if (wg != 0) return;
+  {
+    EndIo io{W, P.words + kWStarted, step_tag(seq, kLayers, kPhStarted), vec};
+    if (!step_may_end(io, pos_raw, P.max_seq, P.advance != 0)) return;
+  }
   if (P.head) {
     if (!W.wait(P.words + kWArg, 2 * kVocabWgs, tag_arg, vec)) return;
     STAMP(kLayers, 3);

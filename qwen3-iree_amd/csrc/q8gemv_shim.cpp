@@ -7,6 +7,7 @@
 #include "qwen3_decode.h"
 #include "prefill_split.h"
 #include "shim_internal.h"
+#include "step_roles.h"
 
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
@@ -49,8 +50,6 @@ constexpr KindInfo kKinds[5] = {
 };
 
 constexpr int kVocabMaxWorkgroups = 8192;
-constexpr int kStepWorkgroups = 448;  // dec_step's workgroups with a role at any context
-constexpr int kStepGrid = 512;        // its launch: two workgroups per CU (long contexts)
 constexpr uint32_t kDefaultSpinLimit = 1u << 20;  // dec_step: poll rounds before a wait gives up
 constexpr int kQ8MaxWorkgroups = 65536;
 constexpr int64_t kBatchWavesPerCu = 10;  // q8gemv_batch default
@@ -1253,7 +1252,7 @@ constexpr size_t kScrStarted = 128;  // u32 the last launch whose grid was resid
 // the attention partials once (layout in decode_kernels.hip)
 constexpr size_t kStepWordsParity = 4 * 512 + 1024 + 512 + 512 + 16 * 16 * 130 + 4 * 1024 +
                                     4 * 512 + 4 * 1536;
-constexpr size_t kStepWords = 2 * kStepWordsParity + 2 * kStepWorkgroups;
+constexpr size_t kStepWords = 2 * kStepWordsParity + 2 * kStepWgs + kStepExtra;
 constexpr size_t kScrWords = (kScrPart + 16 * kAttnGroupsHost * 132 * 4 + 255) / 256 * 256;
 constexpr size_t kScrBytes = kScrWords + kStepWords * 8;
 
