@@ -789,11 +789,7 @@ void dec_step(StepParams P) {
   }
   const int pos_c = pos_raw < 0 ? 0 : (pos_raw >= P.max_seq ? P.max_seq - 1 : pos_raw);
   const bool long_ctx = step_long(pos_c);
-  // Workgroups start in index order: the last one of those every context needs
-  // marks the launch as
-  // resident (a wait that finds another number after ~1 ms knows the grid
-  // is not resident at once).
-  if (wg == kStepWgs - 1 && t == 0)
+  if (wg == step_last_wg(long_ctx) && t == 0)
     __hip_atomic_store(P.last_started, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int tok = *P.token_in;
   tok = (tok < 0 || tok >= kVocab) ? 0 : tok;

@@ -29,6 +29,12 @@ constexpr int kAttnShortCtx = 2048;
 // at position pos (the context is pos + 1)
 constexpr bool step_long(int pos) { return pos >= kAttnShortCtx; }
 
+// The last workgroup a step depends on.  Workgroups start in index order, so once
+// it runs the whole of the step is resident; it marks the launch as such, and a
+// wait that finds the mark missing after about a millisecond gives up instead
+// of polling to its limit.
+constexpr int step_last_wg(bool is_long) { return (is_long ? kStepGrid : kStepWgs) - 1; }
+
 // Whether the step at position pos leaves it on the other side of the switch.
 constexpr bool step_crosses(int pos, int max_seq, bool advance) {
   return advance && pos + 1 < max_seq && !step_long(pos) && step_long(pos + 1);

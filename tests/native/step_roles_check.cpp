@@ -68,7 +68,30 @@ static int run(int pos, int max_seq, bool advance, int n_late, int n_between, bo
   return wrong;
 }
 
+// The device holds the first `resident` workgroups of the launch: whether the
+// mark is there, and whether every workgroup with a role is.
+static bool check_mark(int pos, int resident) {
+  bool marked = false;
+  int roles = 0, running = 0;
+  for (int wg = 0; wg < kStepGrid; ++wg) {
+    const bool role = wg < kStepWgs || step_long(pos);
+    roles += role;
+    if (wg >= resident) continue;
+    running += role;
+    if (wg == step_last_wg(step_long(pos))) marked = true;
+  }
+  if (marked != (running == roles)) {
+    std::printf("pos=%d: %d of the launch resident, %d of %d with a role, marked %d\n", pos,
+                resident, running, roles, marked);
+    return false;
+  }
+  return true;
+}
+
 int main() {
+  for (int pos : {0, kAttnShortCtx - 1, kAttnShortCtx, 8 * kAttnShortCtx})
+    for (int resident = 0; resident <= kStepGrid; ++resident)
+      if (!check_mark(pos, resident)) return 1;
   const int s = kAttnShortCtx;
   const int positions[] = {-5, 0, 1, s - 2, s - 1, s, s + 1, 3 * s, 3 * s + 7};
   const int caches[] = {1, s - 1, s, s + 1, s + 2, 3 * s + 8};

@@ -9,7 +9,8 @@ exits normally) instead of provoking a real stall.  What must hold:
   * qwen3_generate, qwen3_prefill and qwen3_decode_step_checked re-run the
     steps that did nothing with the per-phase launches and return the tokens,
     positions, logits and cache rows of a per-phase run, bit for bit, with
-    status bit 2 and the process-wide fallback count recording it;
+    status bit 2 and the process-wide fallback count recording it, also around
+    and above the context from which the step has 64 more workgroups;
   * single-launch steps of two sessions on two streams, enqueued interleaved,
     are ordered by the library and give each session's bits.
 """
@@ -161,6 +162,43 @@ def test_step_checked_reruns_per_phase(D, dmodel, single):
     assert np.array_equal(got[1], want[1])
     assert got[2] & 4 and not got[2] & 2
     assert D.step_fallback_count() == n0 + 1
+
+
+@pytest.mark.parametrize("pos,after", [(2046, 1), (2046, 2), (2046, None), (3000, 1)])
+def test_generate_resumes_where_the_splits_change(D, dmodel, single, pos, after):
+    """Five tokens from position 2046 (the second step moves the position over
+    the switch and waits for its late workgroups; later ones use all 512) and
+    above it, with the step `after` forced to give up, or none."""
+    rng = np.random.default_rng(pos)
+    k = rng.standard_normal((pos, 1024)).astype(np.float16)
+    v = (0.6 * rng.standard_normal((pos, 1024))).astype(np.float16)
+
+    def run():
+        s = D.DecodeSession(dmodel, pos + 8)
+        for layer in range(28):
+            s.k_cache.upload(np.roll(k, layer, 0), layer * s.max_seq * 2048)
+            s.v_cache.upload(np.roll(v, layer, 0), layer * s.max_seq * 2048)
+        s.set_state(321, pos)
+        toks = s.generate(5, eos_id=-1).tolist()
+        st = s.get_state()
+        cache = [r.view(np.uint16).copy() for layer in (0, 13, 27)
+                 for r in s.cache_rows(layer, pos, s.max_seq)]
+        status = s.check_status()
+        s.free()
+        return toks, st, cache, status
+
+    want = in_mode(D, 0, run)
+    n0 = D.step_fallback_count()
+    if after is not None:
+        D.force_step_abort(after)
+    print(f"generate 5 from position {pos}, give-up at launch {after}", flush=True)
+    got = run()
+    D.force_step_abort(-1)
+    assert got[0] == want[0]
+    assert got[1] == want[1] == (want[0][-1], pos + 5)
+    assert same_cache(got[2], want[2])
+    assert not got[3] & 2 and (got[3] & 4 != 0) == (after is not None)
+    assert D.step_fallback_count() == n0 + (after is not None)
 
 
 def test_two_streams_interleaved(gpu, D, dmodel, single):
