@@ -110,12 +110,12 @@ int qwen3_step_fallback_count(uint64_t* count);
 int qwen3_debug_force_step_abort(int64_t after);
 
 /* How qwen3_decode_step, qwen3_prefill and qwen3_generate run a step:
- * mode 1 = one launch per step (dec_step: all phases in one kernel, 448
- * workgroups, 512 above 2048 positions, resident at once handing activations over through tagged
- * words), the default where the device holds them; mode 0 = one launch per
- * phase (143 per step).  Both
- * compute every value with the same operations in the same order (tested bit
- * for bit).  Setting mode 1 on a device that cannot run it fails with
+ * mode 1 = one launch per step (dec_step: all phases in one kernel, handing
+ * activations over through tagged words; 448 workgroups resident at once up
+ * to 2048 positions, 512 above, launched where max_seq > 2048), the default
+ * where the device holds 448; a step whose grid the device does not hold runs
+ * as in mode 0.  Mode 0 = one launch per phase (143 per step).  Both compute
+ * every value with the same operations in the same order (tested bit for bit).  Setting mode 1 on a device that cannot run it fails with
  * Q8_ERR_BAD_ARGUMENT.  Single-launch steps on different streams run one
  * after another (the library orders each launch after the previous one on
  * any other stream with an event), since two such grids

@@ -139,7 +139,7 @@ struct State {
   std::atomic<int> pf_tile_rows{0};   // prefill GEMM token tile: 0 = by shape, 32, 64 or 128
   std::atomic<int> pf_attn_split{0};  // prefill attention positions per split in blocks of 32
   std::atomic<int> step_single{-1};   // single-launch decode step: -1 unknown, 0 off, 1 on
-  bool step_capable = false;
+  int64_t step_slots = 0;  // dec_step workgroups the device holds at once
   // poll rounds before a dec_step wait gives up
   std::atomic<uint32_t> step_spin_limit{kDefaultSpinLimit};
   // Single-launch steps of different streams run one after another: each
@@ -438,7 +438,7 @@ int q8gemv_init(const char* code_object_path) {
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
-  // The single-launch step needs its 512 workgroups resident together (they
+  // The single-launch step needs its workgroups resident together (they
   // wait on each other's tagged words; there is no grid barrier): a device
   // whose CUs hold them all at once (two per CU), checked from the kernel's
   // occupancy.  It is launched as an ordinary kernel: a cooperative launch
@@ -447,16 +447,16 @@ int q8gemv_init(const char* code_object_path) {
   // kernel on another stream keep some of the workgroups from starting, the
   // bounded waits of the resident ones give up and the step reports status
   // bit 1 (every workgroup then exits) instead of hanging.
-  g.step_capable = false;
+  g.step_slots = 0;
   if (g.dec_step) {
     int per_cu = 0;
     if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, g.dec_step, 256, 0) ==
         hipSuccess)
-      g.step_capable = per_cu >= 1 && (int64_t)per_cu * cus >= kStepGrid;
+      g.step_slots = (int64_t)per_cu * cus;
   }
   // The single launch is the default where it can run: no kernel boundaries,
   // and every workgroup requests its next weights before it waits.
-  if (g.step_single.load() < 0) g.step_single = g.step_capable ? 1 : 0;
+  if (g.step_single.load() < 0) g.step_single = g.step_slots >= kStepWgs ? 1 : 0;
   g.module = mod;
   g.device = dev;
   g.compute_units = cus;
@@ -481,7 +481,7 @@ void q8gemv_shutdown(void) {
   g.dec_module = nullptr;
   g.dec_embed = g.dec_qkv = g.dec_attn = g.dec_o = g.dec_gu = g.dec_dn =
       g.dec_vocab = g.dec_final = g.dec_adv = g.dec_clear = g.dec_step = nullptr;
-  g.step_capable = false;
+  g.step_slots = 0;
   {
     std::lock_guard<std::mutex> step_lock(g.step_mu);
     if (g.step_ev) (void)hipEventDestroy(g.step_ev);
@@ -1334,11 +1334,12 @@ int launch_step(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
   if (g.force_abort_in.load(std::memory_order_relaxed) >= 0 && g.force_abort_in.fetch_sub(1) == 0)
     p.spin_limit = 0;  // the test hook: workgroup 0 gives up at its start
   void* args[] = {&p};
+  const uint32_t grid = (uint32_t)step_grid(max_seq);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(st, &cs));
   if (cs != hipStreamCaptureStatusNone) {
-    hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepGrid, 1, 1, 256, 1, 1, 0, st,
-                                         args, nullptr);
+    hipError_t e = hipModuleLaunchKernel(g.dec_step, grid, 1, 1, 256, 1, 1, 0, st, args,
+                                         nullptr);
     if (e != hipSuccess) return hip_fail(e, "launch of dec_step");
     return Q8_OK;
   }
@@ -1350,7 +1351,7 @@ int launch_step(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
     HIP_TRY(hipEventCreateWithFlags(&g.step_ev, hipEventDisableTiming | hipEventDisableSystemFence));
   else if (g.step_last != st)
     HIP_TRY(hipStreamWaitEvent(st, g.step_ev, 0));
-  hipError_t e = hipModuleLaunchKernel(g.dec_step, kStepGrid, 1, 1, 256, 1, 1, 0, st, args,
+  hipError_t e = hipModuleLaunchKernel(g.dec_step, grid, 1, 1, 256, 1, 1, 0, st, args,
                                        nullptr);
   if (e != hipSuccess) return hip_fail(e, "launch of dec_step");
   HIP_TRY(hipEventRecord(g.step_ev, st));
@@ -1358,9 +1359,11 @@ int launch_step(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t ma
   return Q8_OK;
 }
 
-bool use_single() {
-  return g.step_single.load(std::memory_order_relaxed) == 1 && g.step_capable &&
-         g.dec_step != nullptr;
+// Whether a step over a cache of max_seq positions runs as one launch: the mode
+// asks for it and the device holds the grid (per phase otherwise, the same bits).
+bool use_single(int64_t max_seq) {
+  return g.step_single.load(std::memory_order_relaxed) == 1 && g.dec_step != nullptr &&
+         g.step_slots >= step_grid(max_seq);
 }
 
 // Status bit 1 of a scratch: a single-launch step gave up waiting for a
@@ -2098,9 +2101,9 @@ int qwen3_set_step_mode(int mode) {
   if (mode != 0 && mode != 1) return fail(Q8_ERR_BAD_ARGUMENT, "step mode %d not in {0, 1}", mode);
   int rc = check_decode_ready();
   if (rc) return rc;
-  if (mode == 1 && !g.step_capable)
+  if (mode == 1 && g.step_slots < kStepWgs)
     return fail(Q8_ERR_BAD_ARGUMENT, "this device cannot run the single-launch step "
-                "(needs its 512 workgroups resident at once, two per CU)");
+                "(needs its 448 workgroups resident at once, two per CU)");
   std::lock_guard<std::mutex> lock(g.mu);
   g.step_single = mode;
   return Q8_OK;
@@ -2146,7 +2149,7 @@ int qwen3_get_step_mode(int* mode) {
   if (!mode) return fail(Q8_ERR_NULL_POINTER, "null mode");
   int rc = check_decode_ready();
   if (rc) return rc;
-  *mode = use_single() ? 1 : 0;
+  *mode = use_single(1) ? 1 : 0;
   return Q8_OK;
 }
 
@@ -2212,7 +2215,7 @@ int qwen3_decode_step(const qwen3_weights* w, void* k_cache, void* v_cache, int6
   if (logits && !aligned(logits, 2)) return fail(Q8_ERR_MISALIGNED, "logits 2-byte alignment");
   if ((rc = check_decode_ready())) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (use_single())
+  if (use_single(max_seq))
     return launch_step(w, k_cache, v_cache, max_seq, token, token, pos, logits, nullptr, advance,
                        1, scratch, st);
   void* h = nullptr;
@@ -2229,7 +2232,7 @@ int qwen3_decode_step_checked(const qwen3_weights* w, void* k_cache, void* v_cac
   if ((rc = check_decode_ready())) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if ((rc = check_not_aborted(scratch, st, "before qwen3_decode_step_checked"))) return rc;
-  if (use_single()) {
+  if (use_single(max_seq)) {
     if ((rc = launch_step(w, k_cache, v_cache, max_seq, token, token, pos, logits, nullptr,
                           advance, 1, scratch, st)))
       return rc;
@@ -2260,7 +2263,7 @@ int qwen3_prefill(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t 
   void* status = mb(scratch) + kScrStatus;
   int ms = (int)max_seq;
   int32_t i0 = 0;  // the first prompt token the per-phase launches take
-  if (use_single()) {
+  if (use_single(max_seq)) {
     // the position before and after, so a step that gave up can be resumed
     int32_t p0 = 0, p1 = 0;
     HIP_TRY(hipMemcpyAsync(&p0, pos, sizeof(p0), hipMemcpyDeviceToHost, st));
@@ -2358,7 +2361,7 @@ int qwen3_generate(const qwen3_weights* w, void* k_cache, void* v_cache, int64_t
   uint32_t* status = reinterpret_cast<uint32_t*>(mb(scratch) + kScrStatus);
   // the step mode, once for the call; per-phase for the rest of it after a
   // single launch gave up
-  bool single = use_single();
+  bool single = use_single(max_seq);
   // steps first + from .. first + count - 1 of a batch (from = 0: all)
   auto launch_batch = [&](int32_t first, int32_t count, int slot, int32_t from) -> int {
     for (int32_t b = from; b < count; ++b) {

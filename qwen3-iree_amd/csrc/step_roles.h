@@ -29,6 +29,12 @@ constexpr int kAttnShortCtx = 2048;
 // at position pos (the context is pos + 1)
 constexpr bool step_long(int pos) { return pos >= kAttnShortCtx; }
 
+// Workgroups launched over a cache of max_seq positions: the extra ones only where
+// some step can need them.
+constexpr int step_grid(int64_t max_seq) {
+  return max_seq > kAttnShortCtx ? kStepGrid : kStepWgs;
+}
+
 // The last workgroup a step depends on.  Workgroups start in index order, so once
 // it runs the whole of the step is resident; it marks the launch as such, and a
 // wait that finds the mark missing after about a millisecond gives up instead

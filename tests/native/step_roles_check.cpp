@@ -88,7 +88,21 @@ static bool check_mark(int pos, int resident) {
   return true;
 }
 
+// A step at any position of a cache has the workgroups of its roles, and waits
+// for late ones only where they are launched.
+static bool check_grid(int max_seq) {
+  for (int pos = 0; pos < max_seq; ++pos)
+    if (step_last_wg(step_long(pos)) >= step_grid(max_seq) ||
+        (step_crosses(pos, max_seq, true) && step_grid(max_seq) != kStepGrid)) {
+      std::printf("pos=%d max_seq=%d: grid of %d\n", pos, max_seq, step_grid(max_seq));
+      return false;
+    }
+  return step_grid(max_seq) == (step_long(max_seq - 1) ? kStepGrid : kStepWgs);
+}
+
 int main() {
+  for (int max_seq : {1, kAttnShortCtx - 1, kAttnShortCtx, kAttnShortCtx + 1, 20000})
+    if (!check_grid(max_seq)) return 1;
   for (int pos : {0, kAttnShortCtx - 1, kAttnShortCtx, 8 * kAttnShortCtx})
     for (int resident = 0; resident <= kStepGrid; ++resident)
       if (!check_mark(pos, resident)) return 1;
