@@ -112,7 +112,7 @@ int qwen3_debug_force_step_abort(int64_t after);
 /* How qwen3_decode_step, qwen3_prefill and qwen3_generate run a step:
  * mode 1 = one launch per step (dec_step: all phases in one kernel, handing
  * activations over through tagged words; 448 workgroups resident at once up
- * to 2048 positions, 512 above, launched where max_seq > 2048), the default
+ * to 1280 positions, 512 above, launched where max_seq > 1280), the default
  * where the device holds 448; a step whose grid the device does not hold runs
  * as in mode 0.  Mode 0 = one launch per phase (143 per step).  Both compute
  * every value with the same operations in the same order (tested bit for bit).  Setting mode 1 on a device that cannot run it fails with

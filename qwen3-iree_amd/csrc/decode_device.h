@@ -18,14 +18,14 @@ constexpr int kQHeads = 16;
 constexpr int kFfn = 3072;
 constexpr int kVocab = 151936;
 // Position splits per kv head (one wave each): 32 up to a context of
-// kAttnShortCtx, where a split is at most two chunks of 32 positions; 64 above, where
+// kAttnShortCtx (step_roles.h), 64 above, where
 // the attention is bound by the bytes the waves have in flight (32 splits: 256
 // waves x 16 KiB, 1.63 us per chunk and wave, 2.6 TB/s).  Single-launch step
-// with 32 -> 64 splits, context 2049 / 4096 / 8192 / 16384: 618 -> 607, 673 ->
-// 632, 855 -> 745, 1219 -> 999 us; one layer's launches at 16384 40.2 -> 33.8.
-// At 1025 / 1536 / 2048 64 splits measured 568 / 570 / 573 against 559 / 571 /
-// 586 a step but 25.2-25.6 against 24.1-24.3 a layer (twice the partials to
-// merge).  Two chunks ahead with K rows straight to registers, without more
+// with 32 -> 64 splits, context 1060 / 1150 / 1200 / 1250 / 1300 / 1400: 561.0 ->
+// 564.7, 562.8 -> 564.6, 565.0 -> 565.1, 567.0 -> 565.2, 566.7 -> 564.7, 570.4
+// -> 565.7 us; 1600 / 2048: 574.2 -> 565.6, 591.4 -> 569.0; 4096 / 8192 / 16384:
+// 673 -> 632, 855 -> 745, 1219 -> 999.  One layer's launches: 24.0 -> 24.5 at
+// 1200-2048 (twice the partials to merge), 40.2 -> 33.8 at 16384.  Two chunks ahead with K rows straight to registers, without more
 // waves, was slower (1331 at 16384: the gathered row loads).
 constexpr int kAttnSplits = 32;
 constexpr int kAttnWaves = 4;        // splits per workgroup, merged in LDS

@@ -312,7 +312,7 @@ extern "C" __global__ __launch_bounds__(256) void dec_scratch_clear(uint32_t* __
 // ======================================================= single launch ====
 //
 // dec_step: the whole decode step in one launch of 448 workgroups x 256 threads,
-// 512 over a cache of more than 2048 positions (the last 64 have a role where
+// 512 over a cache of more than 1280 positions (the last 64 have a role where
 // the context is long, see step_roles.h), two per CU, all resident at once (the
 // launcher checks the occupancy; there is no grid barrier, and every wait is
 // bounded).  Work

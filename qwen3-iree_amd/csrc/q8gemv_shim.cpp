@@ -1223,7 +1223,7 @@ constexpr int kLayers = 28;
 constexpr int kVocabRows = 151936;
 constexpr int64_t kKvRow = 8 * 128;  // f16 elements per cache slot
 constexpr int kKvHeads = 8;
-// attention workgroups (partials) per kv head at most: 16 above 2048 positions, else 8
+// attention workgroups (partials) per kv head at most: 16 above kAttnShortCtx positions, else 8
 constexpr int kAttnGroupsHost = 16;
 constexpr int32_t kGenerateBatch = 4;  // tokens between EOS checks (qwen3_full.mlir:1412)
 

@@ -24,7 +24,7 @@ constexpr int kStepGrid = 512;
 constexpr int kStepExtra = kStepGrid - kStepWgs;
 // Contexts up to here have 32 attention splits per kv head, longer ones 64
 // (figures beside kAttnSplits in decode_device.h).
-constexpr int kAttnShortCtx = 2048;
+constexpr int kAttnShortCtx = 1280;
 
 // at position pos (the context is pos + 1)
 constexpr bool step_long(int pos) { return pos >= kAttnShortCtx; }

@@ -1,5 +1,5 @@
 """GPU tests of the decode attention where the number of position splits per
-kv head changes: 32 up to a context of 2048 positions, 64 above.
+kv head changes: 32 up to a context of 1280 positions, 64 above.
 
 - One layer's attention over the GPU's own cache against the oracle, at
   contexts on both sides of the change and at ragged ones (uneven splits, the
@@ -32,7 +32,7 @@ def dmodel(gpu, D, model_host):
     m.free()
 
 
-@pytest.mark.parametrize("ctx", [2047, 2048, 2049, 2050, 2081, 3333, 4096, 4097, 6200])
+@pytest.mark.parametrize("ctx", [1279, 1280, 1281, 1282, 1313, 1999, 2047, 2048, 2049, 2050, 2081, 3333, 4096, 4097, 6200])
 def test_layer_attention_where_the_splits_change(O, gpu, D, dmodel, ctx):
     layer, pos = 4, ctx - 1
     rng = np.random.default_rng(ctx)
@@ -62,7 +62,7 @@ def test_layer_attention_where_the_splits_change(O, gpu, D, dmodel, ctx):
         sess.free()
 
 
-@pytest.mark.parametrize("ctx", [2048, 2049, 3333])
+@pytest.mark.parametrize("ctx", [1280, 1281, 2048, 2049, 3333])
 def test_step_modes_bit_identical_where_the_splits_change(gpu, D, dmodel, ctx):
     rng = np.random.default_rng(7 + ctx)
     k = rng.standard_normal((ctx, 1024)).astype(np.float16)

@@ -164,9 +164,9 @@ def test_step_checked_reruns_per_phase(D, dmodel, single):
     assert D.step_fallback_count() == n0 + 1
 
 
-@pytest.mark.parametrize("pos,after", [(2046, 1), (2046, 2), (2046, None), (3000, 1)])
+@pytest.mark.parametrize("pos,after", [(1278, 1), (1278, 2), (1278, None), (3000, 1)])
 def test_generate_resumes_where_the_splits_change(D, dmodel, single, pos, after):
-    """Five tokens from position 2046 (the second step moves the position over
+    """Five tokens from position 1278 (the second step moves the position over
     the switch and waits for its late workgroups; later ones use all 512) and
     above it, with the step `after` forced to give up, or none."""
     rng = np.random.default_rng(pos)
