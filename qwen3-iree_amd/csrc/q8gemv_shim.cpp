@@ -1961,8 +1961,10 @@ int launch_prefill_layer(const qwen3_weights* w, int layer, void* k_cache, void*
     // f16: q, k, v as one [4096, 1024] matrix, a head (128 columns) a tile.
     // Where 64-token tiles give each CU at most one workgroup (512 tokens), the
     // eight-wave one with six stages in LDS: 300 / 512 tokens 60.4 / 63.0 us a
-    // layer against 65.1 / 65.9 (640 tokens 85.4 against 83.8)
-    if (f16l && (int64_t)(n + 63) / 64 * 32 <= g.compute_units)
+    // layer against 65.1 / 65.9 (640 tokens 85.4 against 83.8).  A gemm_rows
+    // setting picks among the others.
+    if (f16l && (int64_t)(n + 63) / 64 * 32 <= g.compute_units &&
+        g.pf_tile_rows.load(std::memory_order_relaxed) == 0)
       rc = launch_gemm_f16({{g.pf_f16_qkv_22p, 64, 128, 64, 0, 512}}, xn, 1024, wq, 1024, 4096,
                            nullptr, 0, nullptr, 0, n, st, nullptr, 1, &out);
     else if (f16l)

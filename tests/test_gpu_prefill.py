@@ -186,13 +186,15 @@ def test_prefill_batched_matches_decode_steps(gpu, D, dmodel, n):
     b.free()
 
 
-@pytest.mark.parametrize("n", [45, 500, 1100])
+@pytest.mark.parametrize("n", [45, 160, 500, 1100])
 def test_prefill_batched_equals_layer_by_layer(gpu, D, dmodel, model_host, n):
     """The whole-prompt call forms each next layer's attention norm inside
-    ffn_down's reduce (pf_res_reduce_norm; K split in many ranges at 45
-    tokens, in two at 500, one range at 1100); layer by layer
-    (qwen3_prefill_layer) runs pf_rmsnorm instead.  Every layer's k/v slots
-    depend on that norm, so they must agree bit for bit."""
+    ffn_down's reduce (pf_res_reduce_norm; K split in many ranges at 160
+    tokens, in two at 500); layer by layer (qwen3_prefill_layer) runs
+    pf_rmsnorm instead.  At 45 tokens (row products) and 1100 (ffn_down in one
+    launch) both run the same norm, and differ in the weight touch and in the
+    RoPE table, made once or per layer.  Every layer's k/v slots depend on
+    these, so they must agree bit for bit."""
     rng = np.random.default_rng(900 + n)
     prompt = rng.integers(0, D.VOCAB, n).astype(np.int32)
     print(f"prefill batched vs layers n {n}", flush=True)
@@ -297,11 +299,12 @@ def test_prefill_batched_cache_edges(gpu, D, dmodel):
     sess.free()
 
 
-@pytest.mark.parametrize("n,p0", [(45, 3), (300, 0), (600, 0), (1030, 0)])
+@pytest.mark.parametrize("n,p0", [(45, 3), (160, 3), (300, 0), (600, 0), (1030, 0)])
 def test_prefill_tile_rows_bit_identical(gpu, D, dmodel, n, p0):
-    """The 32- and 64-token GEMM tiles give the same bits in every stage
-    (attn_o / ffn_down with K in many ranges at 45 and 300 tokens, in two at
-    600, in one range through the reduce at 1030)."""
+    """The 32- and 64-token GEMM tiles, and those chosen by shape, give the same
+    bits in every stage (attn_o / ffn_down with K in many ranges at 160 and 300
+    tokens, in two at 600, in one at 1030; up to 128 tokens the setting has no
+    tiles to choose among)."""
     rng = np.random.default_rng(9100 + n)
     max_seq = max(MAX_SEQ, p0 + n)
     sess = D.DecodeSession(dmodel, max_seq)

@@ -84,10 +84,12 @@ def run_layer(D, dmodel, sess, n, p0, h_in, f16: bool, rows: int):
     return g, sess.cache_rows(5, 0, sess.max_seq)
 
 
-@pytest.mark.parametrize("n,p0", [(1, 0), (45, 3), (300, 0), (600, 0), (1030, 0), (2100, 7)])
+@pytest.mark.parametrize("n,p0", [(1, 0), (45, 3), (160, 3), (300, 0), (512, 0), (600, 0),
+                                  (1030, 0), (2100, 7)])
 def test_prefill_f16_route_bit_identical_to_q8_route(gpu, D, dmodel, n, p0):
     """Every region and cache row: Q8_0 route (default tile) == f16 route at
-    tile rows 0 (by shape), 32, 64 and 128."""
+    tile rows 0 (by shape: among others the six-stage q/k/v kernel at 160 to
+    512 tokens and the one-launch attn_o / ffn_down above), 32, 64 and 128."""
     rng = np.random.default_rng(9300 + n)
     max_seq = p0 + n + 8
     sess = D.DecodeSession(dmodel, max_seq)
