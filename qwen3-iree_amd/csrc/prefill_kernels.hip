@@ -1050,8 +1050,8 @@ PF_GEMM_F16(pf_gemm_f16_part_44k, kEpiPartial, 4, 4, 128, 2)
 #undef PF_GEMM_F16
 // attn_o (32 stages of K) and ffn_down (48) with the residual in the epilogue
 // where one round of workgroups covers the tokens: 64 x 64 tiles (513 to 1024
-// tokens) or 128 x 64 over eight waves (to about 2560), instead of f32 sums to
-// memory and a reduce launch.  C chains: the K ranges the token count calls
+// tokens) or 128 x 64 over eight waves (to 2048; to 2560 in a round and a quarter,
+// 144 KiB of LDS a workgroup), instead of f32 sums to memory and a reduce launch.  C chains: the K ranges the token count calls
 // for (2: the first half's sums kept aside), the bits of the split product and
 // its reduce.  Layer at 640 / 800 / 1280 / 1500 / 1800 / 2048 tokens: 85.3 /
 // 90.1 / 133.9 / 148.0 / 169.8 / 158.1 -> 77.7 / 82.7 / 112.6 / 125.2 / 145.7 /

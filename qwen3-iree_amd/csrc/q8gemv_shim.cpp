@@ -1772,7 +1772,14 @@ int launch_gemm_res(const void* x, int ldx, const void* wl, int K, void* y, cons
   // One round of workgroups that finish their outputs themselves, where there
   // is such a grid (figures beside the kernels; whole prompts of 640 / 1021
   // tokens with other weights each time 2527 / 2922 -> 2336 / 2761 us, ffn_down
-  // alone 2416 / 2823); a norm that follows is the caller's.
+  // alone 2416 / 2823); a norm that follows is the caller's.  The 128 x 64
+  // kernel, one workgroup a CU, also where a second round is at most a quarter
+  // full (2049 to 2560 tokens on 256 CUs): layer of 2049 / 2304 / 2560 tokens
+  // 201 / 226 / 239 us against 210 / 232 / 246 with the split product, prompt of
+  // 2049 5.67 against 5.79 ms.  Fuller second rounds win a layer by itself (2561
+  // / 3072 / 3500 tokens 245 / 277 / 323 against 251 / 280 / 319) but no prompt,
+  // whose weights come from HBM (2560 / 2688 / 3072 tokens 6.78 / 7.01 / 7.76
+  // against 6.79 / 7.00 / 7.60 ms).
   if (wf16 && splits <= 2 && g.pf_tile_rows.load(std::memory_order_relaxed) == 0) {
     const int64_t wgs64 = ((int64_t)M + 63) / 64 * (kN / 64);
     const int64_t wgs128n = ((int64_t)M + 127) / 128 * (kN / 64);
