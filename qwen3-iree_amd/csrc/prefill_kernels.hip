@@ -1037,7 +1037,6 @@ PF_GEMM_F16(pf_gemm_f16_swiglu_44, kEpiSwiGLU, 4, 4, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_swiglu_24, kEpiSwiGLU, 2, 4, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_swiglu_22, kEpiSwiGLU, 2, 2, 64, 2)
 PF_GEMM_F16(pf_gemm_f16_res_22, kEpiResidual, 2, 2, 128, 2)
-PF_GEMM_F16(pf_gemm_f16_res_22k, kEpiResidual, 2, 2, 256, 2)
 PF_GEMM_F16(pf_gemm_f16_res_12k, kEpiResidual, 1, 2, 256, 3)
 PF_GEMM_F16(pf_gemm_f16_part_22, kEpiPartial, 2, 2, 128, 2)
 PF_GEMM_F16(pf_gemm_f16_part_22k, kEpiPartial, 2, 2, 256, 2)
@@ -1127,7 +1126,7 @@ __device__ __forceinline__ void rope_lane(const float* __restrict__ rope, int m,
 // heads 4w .. 4w + 3, k heads 2w, 2w + 1 and v heads 2w, 2w + 1; the six
 // vectors are independent chains in the same wave.  Lane owns dims 2 lane,
 // 2 lane + 1; per vector the same operations as the decode step's attention
-// prologue; the angles come from pf_rope_table.  k_cache, v_cache: the
+// prologue; the angles come from the RoPE table.  k_cache, v_cache: the
 // layer's base ([max_seq, 8, 128]).
 extern "C" __global__ __launch_bounds__(256) void pf_qk_rope_cache(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,

@@ -127,7 +127,7 @@ struct State {
                 pf_f16_qkv_22p = nullptr,
                 pf_f16_sw_46w = nullptr, pf_f16_sw_44 = nullptr, pf_f16_sw_24 = nullptr,
                 pf_f16_sw_22 = nullptr,
-                pf_f16_res_22 = nullptr, pf_f16_res_22k = nullptr, pf_f16_res_12k = nullptr,
+                pf_f16_res_22 = nullptr, pf_f16_res_12k = nullptr,
                 pf_f16_part_22 = nullptr, pf_f16_part_22k = nullptr, pf_f16_part_12k = nullptr,
                 pf_f16_part_44k = nullptr, pf_expand = nullptr;
   // [64 x 64, 128 x 64 tiles][attn_o, ffn_down][K ranges - 1]
@@ -387,7 +387,6 @@ int q8gemv_init(const char* code_object_path) {
                      {&g.pf_f16_sw_24, "pf_gemm_f16_swiglu_24"},
                      {&g.pf_f16_sw_22, "pf_gemm_f16_swiglu_22"},
                      {&g.pf_f16_res_22, "pf_gemm_f16_res_22"},
-                     {&g.pf_f16_res_22k, "pf_gemm_f16_res_22k"},
                      {&g.pf_f16_res_12k, "pf_gemm_f16_res_12k"},
                      {&g.pf_f16_res_pipe[0][0][0], "pf_gemm_f16_res_o_p1"},
                      {&g.pf_f16_res_pipe[0][0][1], "pf_gemm_f16_res_o_p2"},
@@ -501,7 +500,7 @@ void q8gemv_shutdown(void) {
   std::memset(g.pf_rows_gu, 0, sizeof(g.pf_rows_gu));
   std::memset(g.pf_rows_o, 0, sizeof(g.pf_rows_o));
   std::memset(g.pf_rows_dn, 0, sizeof(g.pf_rows_dn));
-  g.pf_f16_res_22 = g.pf_f16_res_22k = g.pf_f16_res_12k = g.pf_f16_part_22 = g.pf_f16_part_22k =
+  g.pf_f16_res_22 = g.pf_f16_res_12k = g.pf_f16_part_22 = g.pf_f16_part_22k =
       g.pf_f16_part_12k = g.pf_f16_part_44k = g.pf_expand = nullptr;
   g.vocab = g.vocab_finalize = g.argmax = g.ws_reset = g.copy = nullptr;
   g.calib_empty = g.calib_handoff = g.calib_chase = g.read = nullptr;
@@ -1797,7 +1796,6 @@ int launch_gemm_res(const void* x, int ldx, const void* wl, int K, void* y, cons
   if (splits == 1 && !(norm_w && g.pf_gemm_part && (size_t)M * kN * 4 <= part_bytes)) {
     if (wf16)
       return launch_gemm_f16({{g.pf_f16_res_22, 64, 64, 128, 2},
-                              {g.pf_f16_res_22k, 64, 64, 256, 1},
                               {g.pf_f16_res_12k, 32, 64, 256, 0}},
                              x, ldx, wf16, K, kN, y, kN, r, kN, M, st);
     return launch_gemm(g.pf_gemm_res, g.pf_gemm_res_m32, x, ldx, wl, K, kN, 64, y, kN, r, kN, 0,
