@@ -25,7 +25,9 @@
 //
 // Numerics follow the decode step op for op (f16 tensors between ops, f32 in
 // sums, norms and transcendental math): the norms, RoPE, SwiGLU and residual
-// adds are the same device functions the decode kernels call.  The GEMMs use
+// adds are the same device functions the decode kernels call, or have the same
+// operations' bits in another form (norm_pair_mix, head_norm_pair and the sums
+// around them).  The GEMMs use
 // the weights @prefill itself reads: the f16 layer matrices the reference's
 // converter makes from a Q8_0 file, f16(scale * q) with the product exact in
 // f32 and rounded once (tools/convert_gguf_to_irpa.py:28-44, 174-199); every
@@ -70,6 +72,32 @@ __device__ __forceinline__ uint32_t norm_pair_mix(uint32_t h2, uint32_t w2, floa
   return pack_f16x2(x, y);
 }
 
+// (x / r) w of an f16 pair, rounded to f16, as head_norm_rope forms it: the
+// quotient correctly rounded, from inv = 1 / r rounded, by one step of Markstein's
+// division (the residual q r - x is exact under fma; equal to x / r for each of
+// the 2^33 pairs of an f16 and an f32 significand).  The residual's sign is the
+// one that keeps the sign of a zero x.  r is finite, the largest float for an
+// infinite one (inv = 0): a finite x then gives the zero x / r is, an infinite
+// one NaN.
+__device__ __forceinline__ uint32_t head_norm_pair(uint32_t h2, uint32_t w2, float r, float inv) {
+  float q0, q1, e0, e1, x, y;
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[1,0,0]" : "=v"(q0) : "v"(h2), "v"(inv));
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+      : "=v"(q1)
+      : "v"(h2), "v"(inv));
+  asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(e0) : "v"(q0), "v"(r), "v"(h2));
+  asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+      : "=v"(e1)
+      : "v"(q1), "v"(r), "v"(h2));
+  q0 = fmaf(-e0, inv, q0);
+  q1 = fmaf(-e1, inv, q1);
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[0,1,0]" : "=v"(x) : "v"(q0), "v"(w2));
+  asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[0,1,0] op_sel_hi:[0,1,0]"
+      : "=v"(y)
+      : "v"(q1), "v"(w2));
+  return pack_f16x2(x, y);
+}
+
 // ------------------------------------------- head norms, RoPE, caches ----
 //
 // What follows the q/k/v product for one head of a tile of tokens: the head's
@@ -78,8 +106,11 @@ __device__ __forceinline__ uint32_t norm_pair_mix(uint32_t h2, uint32_t w2, floa
 // qwen3_full.mlir:1812-1879), RoPE at position start + token (:1060-1130) from
 // the table, and the cache writes (:1979-1983).  Sixteen lanes a row, lane j
 // holding dims 4 j .. + 3 and the dims 64 above, so a RoPE pair is in one lane
-// and the row's square root and reciprocal serve 8 dims a lane: about 110 VALU
-// instructions per 4 rows (one row per wave: 80 per row).  As its own launch
+// and the row's square root and reciprocal serve 8 dims a lane: about 130 VALU
+// instructions per 4 rows (one row per wave: 80 per row).  The bits are
+// head_norm_rope's: squares added in index order, x / rms correctly rounded
+// (against x times a rounded 1 / rms and the dims d and d + 64 first: 300 / 512 /
+// 2048 tokens 61.1 / 60.9 / 146.6 us a layer, the same within 0.3).  As its own launch
 // this read q, k and v back and took 4.8 / 6.2 / 10.6 us at 512 / 1021 / 2048
 // tokens, with 4-5 us for the table's.
 struct QkvOut {
@@ -125,10 +156,14 @@ __device__ __forceinline__ void qkv_rope_rows(const QkvOut& A, const uint8_t* ti
     }
     const u32x4 cs4 = load_global(reinterpret_cast<const u32x4*>(A.rope + (size_t)m * 128) + j);
     const u32x4 sn4 = load_global(reinterpret_cast<const u32x4*>(A.rope + (size_t)m * 128) + 16 + j);
-    const float ss = reduce_row16(sq_tree4_mix(x0.x, x0.y) + sq_tree4_mix(x1.x, x1.y));
-    const float inv = 1.0f / sqrtf(ss / 128.0f + kEps);
-    const uint32_t n0[2] = {norm_pair_mix(x0.x, w0.x, inv), norm_pair_mix(x0.y, w0.y, inv)};
-    const uint32_t n1[2] = {norm_pair_mix(x1.x, w1.x, inv), norm_pair_mix(x1.y, w1.y, inv)};
+    const float ss = reduce_row16(sq_tree4_mix(x0.x, x0.y)) +
+                     reduce_row16(sq_tree4_mix(x1.x, x1.y));  // dims in index order
+    const float root = sqrtf(ss / 128.0f + kEps);
+    const float inv = 1.0f / root, rms = fminf(root, 3.40282347e38f);
+    const uint32_t n0[2] = {head_norm_pair(x0.x, w0.x, rms, inv),
+                            head_norm_pair(x0.y, w0.y, rms, inv)};
+    const uint32_t n1[2] = {head_norm_pair(x1.x, w1.x, rms, inv),
+                            head_norm_pair(x1.y, w1.y, rms, inv)};
     uint32_t o0[2], o1[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {

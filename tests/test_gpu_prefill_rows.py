@@ -135,6 +135,34 @@ def test_head_norms_rope_and_cache(O, gpu, D, dmodel, model_host, n):
             assert (np.abs(f64(got) - f64(want)) <= rope_tol(O, normed, want)).all(), i
 
 
+@pytest.mark.parametrize("f16", [True, False])
+def test_head_rows_do_not_depend_on_the_prompt_length(gpu, D, dmodel, f16):
+    """From 65 tokens on a q or k row is one chain of products over K, so the
+    first tokens' raw rows are the same in longer prompts; so must be what head
+    norm and RoPE make of them, in the row product's epilogue (up to 128 tokens)
+    and the tiled ones'.  Token 5's row is zero."""
+    h_in = (1.5 * np.random.default_rng(4500).standard_normal((1100, 1024))).astype(np.float16)
+    h_in[5] = 0
+    p0, first = 11, 100
+    dmodel.use_prefill_matrices(f16)
+    res = {}
+    try:
+        for n in (first, 129, 300, 700, 1100):
+            print(f"head rows n {n} f16 {f16}", flush=True)
+            sess = D.DecodeSession(dmodel, p0 + n)
+            try:
+                g = sess.prefill_layer(LAYER, h_in[:n], p0, True)
+                res[n] = [g[name][:first] for name in ("q", "k", "v", "q_roped")] + [
+                    r[p0:p0 + first] for r in sess.cache_rows(LAYER, 0, p0 + n)]
+            finally:
+                sess.free()
+    finally:
+        dmodel.use_prefill_matrices(True)
+    for n, rows in res.items():
+        for name, a, b in zip(("q", "k", "v", "q_roped", "k_cache", "v_cache"), rows, res[first]):
+            assert np.array_equal(a.view(np.uint16), b.view(np.uint16)), (n, name)
+
+
 @pytest.mark.parametrize("n", [513, 575, 992, 993, 1024, 1025, 1153, 1920, 1921, 2047, 2560, 2561])
 def test_unsplit_residual_products(gpu, D, dmodel, w64, n):
     """attn_o and ffn_down around the edges of the one-round products with the
