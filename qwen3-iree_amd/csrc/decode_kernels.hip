@@ -811,7 +811,8 @@ void dec_step(StepParams P) {
     constexpr int64_t bpl_gu = (int64_t)(2 * kFfn) * (kHidden / 32 * 34);
     uint8_t* const la = S.ad.wa[wave];
     // kv_touch task of this wave: head wg mod 8, task (wg / 8) * 4 + wave of
-    // that head's 128 = split (task mod 32), chunk 1 + task / 32 (1-4)
+    // that head's 128 = split (task mod splits), chunk 1 + task / splits: 1-4
+    // of 32 splits, 1-2 of 64
     const int touch_task = (wg >> 3) * 4 + wave;
     const int n_split_chunks = attn_chunks(pos_c);
     const int splits_log2 = attn_splits_log2(pos_c), n_splits = 1 << splits_log2;
@@ -847,10 +848,10 @@ void dec_step(StepParams P) {
                   [](float a, int) { return (uint32_t)f32_to_f16_bits(a); });
       STAMP(layer, 2);
       // Splits of more than one chunk (context past 1024): this layer's cache
-      // chunks 1-4 of every split into the L2 of the XCD whose attention
+      // chunks 1-4 (64 splits: 1-2) of every split into the L2 of the XCD whose attention
       // workgroups read them (head wg mod 8), one chunk per wave, about 2 us
       // before the attention copies them (which then hit L2 instead of HBM):
-      // us/token at context 2048 636.6 -> 619.1, 4096 826.7 -> 761.1, 8192
+      // us/token (32 splits) at context 2048 636.6 -> 619.1, 4096 826.7 -> 761.1, 8192
       // 1158.6 -> 1094.6, 16384 1763.7 -> 1714.0, 1024 unchanged.  Touching
       // the later chunks too (two tasks per wave) measured slower (8192:
       // 1123.0, 16384: 1749.1): L2 holds only so much beside the weights.
