@@ -90,3 +90,53 @@ def test_step_modes_bit_identical_where_the_splits_change(gpu, D, dmodel, ctx):
     for x, y in zip(ca, cb):
         for a, b in zip(x, y):
             assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
+
+
+def _filled(D, dmodel, max_seq, pos, stream=None):
+    rng = np.random.default_rng(pos)
+    k = rng.standard_normal((pos, 1024)).astype(np.float16)
+    v = (0.6 * rng.standard_normal((pos, 1024))).astype(np.float16)
+    sess = D.DecodeSession(dmodel, max_seq, stream)
+    for layer in range(28):
+        sess.k_cache.upload(np.roll(k, layer, 0), layer * max_seq * 2048)
+        sess.v_cache.upload(np.roll(v, layer, 0), layer * max_seq * 2048)
+    sess.set_state(1234, pos)
+    return sess
+
+
+@pytest.mark.parametrize("how", ["prompt_steps", "graph"])
+def test_other_ways_over_the_switch(gpu, D, dmodel, how):
+    """Positions 1278 to 1282 as prompt steps (no vocab product before the last)
+    and as replays of one captured step: the bits of eager per-phase steps."""
+    pos, max_seq, n = 1278, 1290, 5
+    prompt = [5, 151935, 17, 0, 42]
+
+    def run(mode):
+        D.set_step_mode(mode)
+        graph = how == "graph" and mode == 1
+        stream = gpu.Stream() if graph else None
+        sess = _filled(D, dmodel, max_seq, pos, stream)
+        try:
+            print(f"{how} from position {pos}, mode {mode}", flush=True)
+            if how == "prompt_steps":
+                sess.prefill(prompt)
+            else:
+                for _ in range(n):
+                    sess.replay() if graph else sess.step(advance=True, logits=False)
+                    sess.synchronize()
+            assert sess.check_status() == 0
+            return sess.get_state(), [r.view(np.uint16).copy() for layer in (0, 13, 27)
+                                      for r in sess.cache_rows(layer, 0, max_seq)]
+        finally:
+            sess.free()
+            if stream is not None:
+                stream.destroy()
+
+    before = D.step_mode()
+    try:
+        (sa, ca), (sb, cb) = run(1), run(0)
+    finally:
+        D.set_step_mode(before)
+    assert sa == sb and sa[1] == pos + n
+    for a, b in zip(ca, cb):
+        assert np.array_equal(a, b)
