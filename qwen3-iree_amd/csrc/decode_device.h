@@ -24,8 +24,8 @@ constexpr int kVocab = 151936;
 // with 32 -> 64 splits, context 1060 / 1150 / 1200 / 1250 / 1300 / 1400: 561.0 ->
 // 564.7, 562.8 -> 564.6, 565.0 -> 565.1, 567.0 -> 565.2, 566.7 -> 564.7, 570.4
 // -> 565.7 us; 1600 / 2048: 574.2 -> 565.6, 591.4 -> 569.0; 4096 / 8192 / 16384:
-// 673 -> 632, 855 -> 745, 1219 -> 999.  One layer's launches: 24.0 -> 24.5 at
-// 1200-2048 (twice the partials to merge), 40.2 -> 33.8 at 16384.  Two chunks ahead with K rows straight to registers, without more
+// 673 -> 632, 855 -> 745, 1219 -> 999.  One layer's launches: even at
+// 1300-2048 (24.0-24.1), 26.4 -> 25.2 at 4096, 40.2 -> 33.3 at 16384.  Two chunks ahead with K rows straight to registers, without more
 // waves, was slower (1331 at 16384: the gathered row loads).
 constexpr int kAttnSplits = 32;
 constexpr int kAttnWaves = 4;        // splits per workgroup, merged in LDS

@@ -181,24 +181,24 @@ extern "C" __global__ __launch_bounds__(256) void dec_o_res(const uint8_t* __res
   // is conditional and the load stays ahead of the GEMV
   const int row = 4 * (4 * blockIdx.x + wave) + ((t & 63) >> 4);
   const _Float16 h_row = as_half(load_global_u16(h + row));
-  // the partials every context has, ahead of the weights: they return first
-  // and are merged while the weights are in flight
+  // the partials ahead of the weights: they return first and are merged while
+  // the weights are in flight; the position arrives while the first 8 groups'
+  // loads are being issued (a layer at 1300-2048 / 4096 / 16384 positions 24.0 /
+  // 25.2 / 33.3 us against 24.4 / 25.6 / 33.7 with groups 8 .. 15 requested
+  // behind the weights; 22.8 at 300 either way)
   const float* ph = part + (size_t)(t >> 4) * kAttnGroupsMax * kPartStride;
   const int d0 = 8 * (t & 15);
   Partials p;
   load_partials<0>(p, ph, d0);
   __builtin_amdgcn_sched_barrier(0);
+  const bool is_long = step_long(pos_raw < max_seq ? pos_raw : max_seq - 1);
+  if (is_long) load_partials<kAttnGroups>(p, ph, d0);
+  __builtin_amdgcn_sched_barrier(0);
   const float acc = q8_quad_core_acc<2>(
       wo, kHidden, 4 * blockIdx.x + wave, lds + wave * LDSB,
       [&](u32x4 (&xr)[2][8]) {
-        const int pos = pos_raw < max_seq ? pos_raw : max_seq - 1;
-        u32x4 packed;
-        if (attn_splits(pos) == kAttnSplits) {
-          packed = merge_partials<kAttnGroups>(p);
-        } else {
-          load_partials<kAttnGroups>(p, ph, d0);
-          packed = merge_partials<kAttnGroupsMax>(p);
-        }
+        const u32x4 packed =
+            is_long ? merge_partials<kAttnGroupsMax>(p) : merge_partials<kAttnGroups>(p);
         reinterpret_cast<u32x4*>(attn)[t] = packed;
         if (blockIdx.x == 0) reinterpret_cast<u32x4*>(attn_out)[t] = packed;
         __syncthreads();
